@@ -21,6 +21,8 @@
 //     positions;
 //   * chunked (small caches, the code predictor, short arenas): one workgroup per (request,
 //     chunk of 64-key blocks, KV head), whose rows are requested together with its position.
+//     bf16 calls over rows of 128 that set no chunk count run unsplit instead, one workgroup per
+//     (request, KV head) (decode_direct.hip; direct_ok).
 // For these two:
 //   * lanes: 16 bytes of one key row per lane (LPK lanes per key); a pass of the workgroup
 //     reads 4 KiB of K and 4 KiB of V, all passes of a block are issued before any math;
@@ -61,15 +63,6 @@ Q3T_DEVICE float lane_dot(const U4 &q, const U4 &k) {
     }
 }
 
-// Sum over each aligned group of LPK (8, 16 or 32) lanes; every lane of the group gets it.
-template <int LPK>
-Q3T_DEVICE float group_sum(float x) {
-    x = sum8(x);
-    if constexpr (LPK >= 16) x += xor8(x);
-    if constexpr (LPK >= 32) x += xor16(x);
-    return x;
-}
-
 // Sum / max across the lane groups of a wave (lanes that differ in the bits above the group).
 template <int LPK>
 Q3T_DEVICE float cross_sum(float x) {
@@ -82,32 +75,6 @@ Q3T_DEVICE float cross_max(float x) {
     if constexpr (LPK <= 8) x = fmaxf(x, xor8(x));
     if constexpr (LPK <= 16) x = fmaxf(x, xor16(x));
     return fmaxf(x, xor32(x));
-}
-
-// RMSNorm of one bf16 row spread over LPK lanes (8 elements per lane), as the attention
-// module's q_norm / k_norm compute it: fp32 sum of squares over the row, x * rsqrt(mean + eps)
-// rounded to bf16, times the bf16 weight, rounded to bf16.  The sum's order is this kernel's
-// (lanes, then the DPP tree); rows agree with other orders to the last bf16 bit except near
-// rounding ties.
-template <int LPK>
-Q3T_DEVICE U4 rms_norm8(const U4 &x, const U4 &w, float eps, int width) {
-    const uint32_t v[4] = {x.x, x.y, x.z, x.w}, g[4] = {w.x, w.y, w.z, w.w};
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = bf16_lo(v[i]), b = bf16_hi(v[i]);
-        ss = __builtin_fmaf(a, a, ss);
-        ss = __builtin_fmaf(b, b, ss);
-    }
-    ss = group_sum<LPK>(ss);
-    const float r = __builtin_amdgcn_rsqf(ss * (1.0f / (float)width) + eps);
-    uint32_t y[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t n = cvt_pk_bf16(bf16_lo(v[i]) * r, bf16_hi(v[i]) * r);
-        y[i] = cvt_pk_bf16_canon(bf16_lo(n) * bf16_lo(g[i]), bf16_hi(n) * bf16_hi(g[i]));
-    }
-    return U4{y[0], y[1], y[2], y[3]};
 }
 
 // Cross-workgroup chunk states are written and read with device-scope (sc1) accesses, which
@@ -124,14 +91,6 @@ Q3T_DEVICE void wait_stores() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);  // all counters zero: every issued store has completed
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-template <typename T>
-Q3T_DEVICE void store_out(char *base, float v) {
-    if constexpr (sizeof(T) == 2)
-        *reinterpret_cast<uint16_t *>(base) = (uint16_t)float_to_bf16(v);
-    else
-        *reinterpret_cast<float *>(base) = v;
 }
 
 // Sums of N values across the lane halves (permlane32_swap) and then across 16-lane rows
@@ -1413,6 +1372,38 @@ static bool bundle_ok(const q3t_decode_args *a) {
     return a->dtype == Q3T_BF16 && a->head_dim == 128 && a->query_len == 1 && bundle_mask_ok(a) &&
            a->batch <= kBundleMaxBatch && a->q_heads / a->kv_heads <= 4;
 }
+// Whether a call on the chunked grid runs unsplit, one workgroup per (request, KV head)
+// (decode_direct.hip): bf16 rows of 128, one or two query tokens, row offsets that fit 32 bits;
+// a mask as the bundled grid takes it.  Callers that set a chunk count, or
+// `splits`, get the split kernel.
+static bool direct_ok(const q3t_decode_args *a) {
+    const int64_t G = a->q_heads / a->kv_heads;
+    if (a->dtype != Q3T_BF16 || a->head_dim != 128 || a->query_len > 2 || (G != 1 && G != 2 && G != 4) ||
+        a->ctx >= kDirectMaxCtx || a->splits != 0 || a->max_chunks > 0)
+        return false;
+    if (!bundle_mask_ok(a) || (a->mask && a->mask_stride_s < 0)) return false;
+    // the whole extent of the rows of a call in 31-bit byte offsets, key rows apart, arena planes in
+    // 32-bit counts of 16 bytes
+    const int64_t B = a->batch, S = a->query_len, Hq = a->q_heads, Hkv = a->kv_heads;
+    const int64_t rows[][6] = {{a->q_stride_b, B, a->q_stride_s, S, a->q_stride_h, Hq},
+                               {a->o_stride_b, B, a->o_stride_s, S, a->o_stride_h, Hq},
+                               {a->nk_stride_b, B, a->nk_stride_s, S, a->nk_stride_h, Hkv},
+                               {a->nv_stride_b, B, a->nv_stride_s, S, a->nv_stride_h, Hkv},
+                               {a->cs_stride_b, B, a->cs_stride_s, S, 0, 1}};
+    const int64_t limit = (int64_t)1 << 30;  // elements: 2 GiB of bytes
+    for (const auto &r : rows) {
+        int64_t extent = 0;
+        for (int i = 0; i < 6; i += 2) {
+            if (r[i] < 0 || r[i] >= limit) return false;
+            extent += r[i] * r[i + 1];
+        }
+        if (extent >= limit) return false;
+    }
+    if (a->k_stride_t < 128 || a->v_stride_t < 128) return false;
+    for (const int64_t st : {a->k_stride_b, a->k_stride_h, a->v_stride_b, a->v_stride_h})
+        if (st < 0 || st / 8 > INT32_MAX) return false;
+    return true;
+}
 static int decode_grid(const q3t_decode_args *a) {
     switch (a->grid) {
         case Q3T_GRID_CHUNKED: return Q3T_GRID_CHUNKED;
@@ -1665,6 +1656,10 @@ static int decode_launch(const q3t_decode_args *a, const DecodeParams &p, void *
     const int g = (int)(a->q_heads / a->kv_heads);
     const int sq = (int)a->query_len;
     const bool fused = a->fused != 0;
+    if (decode_grid(a) == Q3T_GRID_CHUNKED && direct_ok(a)) {
+        direct_launch(p, g, sq, fused, s);
+        return launch_status();
+    }
     int st;
     if (a->dtype == Q3T_BF16)
         st = a->head_dim == 128 ? dispatch_g<uint16_t, 128>(p, g, sq, fused, s)

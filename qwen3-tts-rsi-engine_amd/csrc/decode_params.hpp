@@ -41,6 +41,11 @@ int64_t plan_bundle_count(int64_t batch, int64_t kv_heads);
 int64_t plan_ints(int64_t batch, int64_t kv_heads);
 int plan_launch(const int64_t *pos, int batch, int ctx, int bundles, int32_t *plan, hipStream_t s);
 
+// The unsplit form of the chunked grid (decode_direct.hip): one workgroup per (request, KV head).
+constexpr int kDirectMaxCtx = 2048;    // longest context it takes (a mask row's words in LDS)
+constexpr int kDirectManyPairs = 64;   // (request, KV head) pairs from which its workgroups are smaller
+void direct_launch(const DecodeParams &p, int group, int tokens, bool fused, hipStream_t s);
+
 // 4 bytes per lane from global memory into LDS at lds_base + 4 * lane (the mask words of a
 // stage's rows); offsets past the resource's range write zeros.
 Q3T_DEVICE void load_to_lds4(i32x4_t rsrc, uint32_t voffset, uint32_t lds_base) {
@@ -68,6 +73,49 @@ Q3T_DEVICE float load_mask(const char *m, int dtype) {
         case Q3T_F32: return *reinterpret_cast<const float *>(m);
         default: return *reinterpret_cast<const uint8_t *>(m) ? 0.0f : -INFINITY;  // bool: True attends
     }
+}
+
+// Sum over each aligned group of LPK (8, 16 or 32) lanes; every lane of the group gets it.
+template <int LPK>
+Q3T_DEVICE float group_sum(float x) {
+    x = sum8(x);
+    if constexpr (LPK >= 16) x += xor8(x);
+    if constexpr (LPK >= 32) x += xor16(x);
+    return x;
+}
+
+// RMSNorm of one bf16 row spread over LPK lanes (8 elements per lane), as the attention
+// module's q_norm / k_norm compute it: fp32 sum of squares over the row, x * rsqrt(mean + eps)
+// rounded to bf16, times the bf16 weight, rounded to bf16.  The sum's order is this kernel's
+// (lanes, then the DPP tree); rows agree with other orders to the last bf16 bit except near
+// rounding ties.
+template <int LPK>
+Q3T_DEVICE U4 rms_norm8(const U4 &x, const U4 &w, float eps, int width) {
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w}, g[4] = {w.x, w.y, w.z, w.w};
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = bf16_lo(v[i]), b = bf16_hi(v[i]);
+        ss = __builtin_fmaf(a, a, ss);
+        ss = __builtin_fmaf(b, b, ss);
+    }
+    ss = group_sum<LPK>(ss);
+    const float r = __builtin_amdgcn_rsqf(ss * (1.0f / (float)width) + eps);
+    uint32_t y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t n = cvt_pk_bf16(bf16_lo(v[i]) * r, bf16_hi(v[i]) * r);
+        y[i] = cvt_pk_bf16_canon(bf16_lo(n) * bf16_lo(g[i]), bf16_hi(n) * bf16_hi(g[i]));
+    }
+    return U4{y[0], y[1], y[2], y[3]};
+}
+
+template <typename T>
+Q3T_DEVICE void store_out(char *base, float v) {
+    if constexpr (sizeof(T) == 2)
+        *reinterpret_cast<uint16_t *>(base) = (uint16_t)float_to_bf16(v);
+    else
+        *reinterpret_cast<float *>(base) = v;
 }
 
 }  // namespace q3t

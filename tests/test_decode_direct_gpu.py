@@ -1,0 +1,154 @@
+"""Decode attention with one workgroup per (request, KV head): the chunked grid's unsplit form
+(bf16, head_dim 128, contexts below 2048 rows).
+
+Against the float64 oracle (max-abs <= 2e-2, mean-abs <= 2e-3 for bf16 I/O with fp32
+accumulation) over one, four and eight waves per workgroup, with lengths on and around the
+16-key stages and the workgroup's whole stages, invalid positions, arenas read through
+offsets, and masks of every type that hide keys in the middle, at the end or all but one.
+The weights enter the products with 16 significant bits, so the result is as close to float64
+as the split kernel's float32 weights: its error norm is held to 1.02 times that kernel's."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as oatt
+from oracle import bf16 as obf16
+from oracle import rope as orope
+from tests._util import assert_attention_close, bits, f64
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+# (batch, kv_heads, capacity): one wave; one wave with two stages; four waves (256 pairs);
+# eight waves, one stage to sixteen
+SHAPES = [(9, 8, 16), (5, 4, 32), (40, 8, 33), (64, 8, 300), (3, 8, 33), (7, 8, 130), (2, 2, 512), (5, 4, 1500), (2, 8, 2047)]
+
+
+def _problem(batch, kv_heads, group, capacity, seed, device, tokens=1):
+    gen = torch.Generator(device=device).manual_seed(seed)
+    keys = torch.randn(batch, kv_heads, capacity, D, generator=gen, device=device, dtype=torch.bfloat16)
+    values = torch.randn(keys.shape, generator=gen, device=device, dtype=torch.bfloat16)
+    rows = torch.randn(batch, tokens, kv_heads * (group + 2), D, generator=gen, device=device, dtype=torch.bfloat16)
+    q, k, v = rows.split([kv_heads * group, kv_heads, kv_heads], dim=2)
+    host = torch.Generator().manual_seed(seed)
+    positions = torch.randint(0, capacity, (batch,), generator=host)
+    edge = torch.tensor([capacity - 1, 0, 15, 16, 17, 63, 64, 127, 128, 31, -1, capacity])
+    edge = edge[(edge <= capacity)][:batch - 1]
+    positions[:len(edge)] = edge
+    return keys, values, q, k, v, positions
+
+
+def _valid(positions, capacity):
+    return ((positions >= 0) & (positions < capacity)).numpy()
+
+
+@pytest.mark.parametrize("group", [1, 2, 4])
+@pytest.mark.parametrize("batch,kv_heads,capacity", SHAPES)
+def test_attention_matches_the_oracle_and_the_split_kernel(pkg, device, batch, kv_heads, capacity, group):
+    keys, values, q, _, _, positions = _problem(batch, kv_heads, group, capacity, 3 + capacity, device)
+    assert pkg.decode_grid_for(batch, 1, kv_heads * group, kv_heads, D, capacity) == "chunked"
+    dpos = positions.to(device)
+    out = pkg.decode_attention(q, keys, values, dpos)
+    split = pkg.decode_attention(q, keys, values, dpos, max_chunks=1)
+    offsets = torch.arange(batch, device=device).flip(0) * keys.stride(0)
+    moved = pkg.decode_attention(q, keys, values, dpos, kv_offsets=offsets)
+    flipped = pkg.decode_attention(q, keys.flip(0).contiguous(), values.flip(0).contiguous(), dpos)
+    ok = _valid(positions, capacity)
+    assert bool((out[~torch.from_numpy(ok)] == 0).all())
+    assert torch.equal(moved, flipped)
+    expected = oatt.decode_attention(f64(q), f64(keys), f64(values), np.where(ok, positions.numpy(), 0), D ** -0.5)[ok]
+    assert_attention_close(f64(out)[ok], expected)
+    error, reference = (np.linalg.norm(f64(x)[ok] - expected) for x in (out, split))
+    assert error <= 1.02 * reference
+
+
+@pytest.mark.parametrize("tokens", [1, 2])
+@pytest.mark.parametrize("batch,kv_heads,capacity", SHAPES)
+def test_fused_step(pkg, device, batch, kv_heads, capacity, tokens):
+    """RoPE, the paired write (bit-exact) and the attention, one and two tokens, against the
+    rotated rows written by the oracle."""
+    group = 2
+    keys, values, q, k, v, positions = _problem(batch, kv_heads, group, capacity, 5 + capacity, device, tokens)
+    positions[positions == 0] = tokens - 1  # every token has a position
+    ok = _valid(positions, capacity)
+    at = torch.where(torch.from_numpy(ok), positions, torch.full_like(positions, tokens - 1))
+    where = (at[:, None] - tokens + 1 + torch.arange(tokens)).to(device)
+    cos, sin = pkg.rope_tables(where, D)
+    before_k, before_v = bits(keys).copy(), bits(values).copy()
+    out = pkg.decode_step(q, k, v, keys, values, positions.to(device), cos, sin)
+    cb, sb = bits(cos)[:, :, None, :], bits(sin)[:, :, None, :]
+    q_rot, k_rot = orope.rope_bf16(bits(q), cb, sb), orope.rope_bf16(bits(k), cb, sb)
+    for b in np.flatnonzero(ok):
+        rows = where[b].cpu().numpy()
+        before_k[b][:, rows] = k_rot[b].transpose(1, 0, 2)
+        before_v[b][:, rows] = bits(v)[b].transpose(1, 0, 2)
+    assert np.array_equal(bits(keys), before_k) and np.array_equal(bits(values), before_v)
+    assert bool((out[~torch.from_numpy(ok)] == 0).all())
+    kf, vf, qf = obf16.from_bits(before_k), obf16.from_bits(before_v), obf16.from_bits(q_rot)
+    for t in range(tokens):
+        last = np.where(ok, at.numpy() - tokens + 1 + t, 0)
+        expected = oatt.decode_attention(qf[:, t:t + 1], kf, vf, last, D ** -0.5)[ok]
+        assert_attention_close(f64(out)[ok][:, t:t + 1], expected)
+
+
+@pytest.mark.parametrize("tokens", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bool, torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("batch,kv_heads,capacity", [(6, 8, 30), (33, 8, 131), (3, 8, 515), (2, 4, 2047)])
+def test_masks(pkg, device, batch, kv_heads, capacity, dtype, tokens):
+    """Rows that hide a random half, everything past a prefix, all but the last or the first
+    key, and nothing; odd widths put the rows off their words' boundaries."""
+    group = 2
+    keys, values, q, _, _, _ = _problem(batch, kv_heads, group, capacity, 7 + capacity, device, tokens)
+    gen = torch.Generator().manual_seed(capacity)
+    seen = torch.rand(batch, tokens, capacity, generator=gen) < 0.5
+    seen[..., 0] = True
+    key = torch.arange(capacity)
+    for b in range(batch):
+        for t in range(tokens):
+            kind = (b + t) % 5
+            if kind == 1: seen[b, t] = key <= (37 * b) % capacity
+            if kind == 2: seen[b, t] = key == capacity - 1
+            if kind == 3: seen[b, t] = key == 0
+            if kind == 4: seen[b, t] = True
+    mask = seen if dtype == torch.bool else torch.zeros(seen.shape, dtype=dtype).masked_fill(~seen, torch.finfo(dtype).min)
+    positions = torch.full((batch,), capacity - 1, device=device, dtype=torch.int64)
+    out = pkg.decode_attention(q, keys, values, positions, mask=mask.to(device)[:, None])
+    scores = np.einsum("bshgd,bhnd->bshgn", f64(q).reshape(batch, tokens, kv_heads, group, D), f64(keys)) * D ** -0.5
+    scores = np.where(seen.numpy()[:, :, None, None], scores, -np.inf)
+    weights = np.exp(scores - scores.max(-1, keepdims=True))
+    weights /= weights.sum(-1, keepdims=True)
+    expected = np.einsum("bshgn,bhnd->bshgd", weights, f64(values)).reshape(batch, tokens, -1, D)
+    assert_attention_close(f64(out), expected)
+
+
+def test_a_masked_row_past_the_last_visible_key_is_not_read_and_infinite_values_stay(pkg, device):
+    keys, values, q, _, _, _ = _problem(4, 8, 2, 200, 11, device)
+    mask = (torch.arange(200, device=device) < 50).expand(4, 200)[:, None, None, :].contiguous()
+    positions = torch.full((4,), 199, device=device, dtype=torch.int64)
+    expected = pkg.decode_attention(q, keys, values, positions, mask=mask)
+    again = pkg.decode_attention(q, keys[:, :, :50], values[:, :, :50], torch.full_like(positions, 49))
+    assert torch.equal(expected, again)
+    values[:, :, 3, 5] = float("inf")  # a visible key: the dim is infinite, the others unchanged
+    out = pkg.decode_attention(q, keys, values, positions, mask=mask)
+    assert bool(torch.isposinf(out[..., 5]).all())
+    keep = torch.arange(D, device=device) != 5
+    assert torch.equal(out[..., keep], expected[..., keep])
+
+
+def test_step_in_a_graph_follows_rewritten_positions(pkg, device):
+    keys, values, q, k, v, positions = _problem(6, 8, 2, 300, 13, device)
+    positions = positions.clamp(0, 299).to(device)
+    cos, sin = pkg.rope_tables(positions, D)
+    out = torch.empty_like(q)
+    pkg.decode_step(q, k, v, keys, values, positions, cos, sin, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.inference_mode(), torch.cuda.graph(graph):
+        pkg.decode_step(q, k, v, keys, values, positions, cos, sin, out=out)
+    for step in range(3):
+        positions.copy_((positions * 7 + 13 + step) % 300)
+        keys2, values2 = keys.clone(), values.clone()
+        expected = pkg.decode_step(q, k, v, keys2, values2, positions, cos, sin)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected) and torch.equal(keys, keys2) and torch.equal(values, values2)

@@ -345,6 +345,16 @@ typedef struct q3t_prefill_rope_write_args {
 
 int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *args, void *stream);
 
+/*
+ * One prefill layer: q3t_prefill_rope_write(write, stream), then
+ * q3t_prefill_attention(attend, stream), both validated before anything is launched.  Where the
+ * two describe one step of short requests (the same tokens, tables and arena; keys only in
+ * `write`, new_values in `attend`, no mask or kv_lens, max_seqlen up to 64) a single launch does
+ * the work: the attention rotates the keys as it reads them and writes them into the arena.
+ * Replaces: PrefillGraph.compute's attention layer (prefill_graph.py:38-50).
+ */
+int q3t_prefill_step(const q3t_prefill_rope_write_args *write, const q3t_prefill_args *attend, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -108,6 +108,7 @@ SIGNATURES = {
     "q3t_decode_attention_static": (ctypes.c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
     "q3t_prefill_attention": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), c_vp]),
     "q3t_prefill_rope_write": (ctypes.c_int, [ctypes.POINTER(PrefillRopeWriteArgs), c_vp]),
+    "q3t_prefill_step": (ctypes.c_int, [ctypes.POINTER(PrefillRopeWriteArgs), ctypes.POINTER(PrefillArgs), c_vp]),
 }
 
 _lock = threading.Lock()

@@ -469,6 +469,18 @@ def prefill_attention(query, keys, values, cu_seqlens, max_seqlen, *, scale=None
     (``prefill_rope_write(value=None)`` left them out of the arena): the products read them
     and the same launch copies each into ``values`` at its token's position.  Not with
     ``mask``."""
+    a, out, device, kept = prefill_args(query, keys, values, cu_seqlens, max_seqlen, scale, kv_slots, out, cos, sin,
+                                        kv_lens, mask, new_values)
+    status = _lib.library().q3t_prefill_attention(a, _lib.stream_handle(device))
+    del kept
+    _lib.check(status, 'prefill attention')
+    return out
+
+
+def prefill_args(query, keys, values, cu_seqlens, max_seqlen, scale, kv_slots, out, cos, sin, kv_lens, mask, new_values):
+    """The validated arguments of ``prefill_attention``: (arguments, out, device, a tensor made
+    here that the launch reads, or None)."""
+    kept = None
     if query.ndim != 3 or keys.ndim != 4 or values.shape != keys.shape:
         raise ValueError('expected (T, Hq, D) queries and arena key/value views')
     total, q_heads, head_dim = query.shape
@@ -534,9 +546,8 @@ def prefill_attention(query, keys, values, cu_seqlens, max_seqlen, *, scale=None
         a.mask = m.data_ptr()
         a.mask_dtype = _lib.DTYPE_CODES[m.dtype]
         a.mask_stride_b, a.mask_stride_q = m.stride(0), m.stride(2)
-    status = _lib.library().q3t_prefill_attention(a, _lib.stream_handle(device))
-    _lib.check(status, 'prefill attention')
-    return out
+        kept = m
+    return a, out, device, kept
 
 
 def _prefill_mask(mask, batch, queries, keys):

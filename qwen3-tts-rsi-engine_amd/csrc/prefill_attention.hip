@@ -116,37 +116,46 @@ __global__ void __launch_bounds__(256) prefill_rope_write_kernel(PrefillRopeWrit
 
 // ---- varlen causal attention on bf16 MFMA tiles ------------------------------------------
 //
-// One workgroup of 4 waves per (request, 64-query block, GH query heads of one KV head);
-// wave w owns queries q0 + 16w ... q0 + 16w + 15 of every one of the GH heads, so each K and
-// V read from LDS feeds the products of all GH heads (GH = 2: 168 VGPRs, 3 waves per SIMD,
-// every workgroup of the 16-prompt workload resident at once).  Keys stream through
-// a ring of kStages LDS stages of kTile keys (K rows then V rows), filled by buffer loads
-// that write LDS directly (16 bytes per lane) kStages - 1 tiles ahead of the products, so
-// the K/V reads never pass through registers.  Rows are stored unpadded with their 16-byte
-// chunks XOR-swizzled (K chunk ch of row r at ch ^ (r & 15), V at ch ^ (2r & 15)), which
-// keeps the 16-byte K reads of 16 rows and the transposing 8-byte V reads of 8 rows on
-// distinct banks.  With v_mfma_f32_16x16x32_bf16 (lane l = 16g + c holds A[c][8g..8g+7],
-// B[8g..8g+7][c] and D[4g..4g+3][c]), per 32 keys:
-//   S^T (keys x queries) = K . Q^T   A = K rows from LDS, B = the wave's Q rows (registers);
-//                                    lane (g, c) gets keys 4g..4g+3 and 16+4g..16+4g+3 of
-//                                    query c;
-//   O^T (dims x queries) += V^T . P^T   B = P^T straight from the S^T registers (K index
-//                                    order {4g..4g+3, 16+4g..16+4g+3}); A = V^T read by
-//                                    ds_read_b64_tr_b16: within a 16-lane group, lane c reads
-//                                    4 dims of key row 4g + c/4 and receives, after the
-//                                    transpose, keys 4g..4g+3 of dim c.
-// Each lane keeps the online-softmax state of one query per head.  The causal mask is applied only
-// on the steps that straddle the wave's diagonal or the end of the keys.  The running
-// maximum moves only when a step's maximum exceeds it by more than kRescaleLog2 (log2
-// units), so the accumulators are rescaled rarely and unnormalised weights stay below
-// 2^kRescaleLog2 (well inside bf16 and fp32 range).
-constexpr int kQBlock = 64;
+// One workgroup of 4 waves per (request, query block, GH query heads of one KV head).  A wave
+// owns 32 columns: with GH = 2 the two heads' rows of 16 queries (64-query blocks), with GH = 1
+// 32 queries of one head (128-query blocks); every K and V row read from LDS feeds all 32.
+// Keys stream through a ring of kStages LDS stages of kTile keys (K rows then V rows), filled by
+// buffer loads that write LDS directly (16 bytes per lane) kStages - 1 tiles ahead of the
+// products, so the K/V reads never pass through registers.  With v_mfma_f32_32x32x16_bf16 (lane
+// l = 32 hi + c holds A[c][8 hi ... 8 hi + 7], B[8 hi ... 8 hi + 7][c] and D[8 i + 4 hi ... + 3][c],
+// i = 0..3), per 32 keys:
+//   S^T (keys x columns) = K . Q^T   A = K rows from LDS, B = the wave's query rows (registers);
+//                                    lane (hi, c) gets keys 8 i + 4 hi + {0..3} of column c;
+//   O^T (dims x columns) += V^T . P^T   B = P^T straight from the S^T registers (contraction
+//                                    order, per 16 keys: 4 hi + {0..3}, 8 + 4 hi + {0..3}); A = V^T
+//                                    read by ds_read_b64_tr_b16 in that order: within a 16-lane
+//                                    group, lane i reads 4 dims of key row i/4 and receives, after
+//                                    the transpose, 4 keys of dim i.
+// A lane keeps the online softmax of one column, and one column's keys sit in two lanes, so a
+// step costs one maximum, one threshold and one sum per lane and 24 LDS reads for 16 products.
+// (The same tiles as 16x16x32 products, a head after the other, took 40 LDS reads, 32 products and
+// two softmax states per step.)
+// What bounds it: where the launch fills the card, memory and the workgroups' start as much as the
+// products (16 prompts of 32..512 with no tile at all: 19 of 25.8 us, the query, value and output
+// rows at ~3.6 TB/s); where it does not, the longest block's chain of tiles.  us per layer for the
+// whole step, before -> after this form: one prompt of 464 22.1 -> 17.9, of 2048 66.8 -> 45.1, 4 of
+// 100..300 20.3 -> 17.4, 8 x 256 under a mask 21.1 -> 17.2, 32 of 500 102 -> 94.7, 16 of 32..512 32.7 ->
+// 32.2.
+// Rows are stored unpadded with their 16-byte chunks XOR-swizzled (K chunk ch of row r at
+// ch ^ (r & 15), V at ch ^ 4 (r & 3) for rows of 256 bytes), which keeps the 16-byte K reads of
+// 32 rows and the transposing V reads of 4 rows x 64 bytes on distinct banks.
+// The causal mask is applied only on the steps that straddle the wave's diagonal or the end of
+// the keys.  The running maximum moves only when a step's maximum exceeds it by more than
+// kRescaleLog2 (log2 units), so the accumulators are rescaled rarely and unnormalised weights
+// stay below 2^kRescaleLog2 (well inside bf16 and fp32 range).
 constexpr int kXcds = 8;        // MI355X: 8 XCDs of 32 CUs
 constexpr int kCusPerXcd = 32;
-constexpr int kTile = 32;     // keys per LDS stage and per softmax step
-constexpr int kStages = 3;    // LDS ring depth: loads run kStages - 1 tiles ahead
+constexpr int kKeys = 32;     // keys of one MFMA block of scores
 constexpr float kLog2eP = 1.4426950408889634f;
 constexpr float kRescaleLog2 = 8.0f;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+// Queries per workgroup.
+constexpr int query_block(int gh) { return 4 * (32 / gh); }
 
 struct PrefillParams {
     int B, Hq, Hkv, nqb, group;
@@ -170,75 +179,16 @@ struct PrefillParams {
     int mdt;              // mask element type (Q3T_BF16, Q3T_F16 or Q3T_F32)
     int64_t m_sb, m_sq;   // mask strides (elements) of requests and query rows; keys unit-stride
     // optional value rows of the step's tokens as the projection wrote them: the products
-    // read them (key j of request b is token cu[b] + j) and the workgroups past the
-    // attention grid copy them into the arena view `v` at each token's position
+    // read them (key j of request b is token cu[b] + j) and each workgroup copies those of its
+    // query block into the arena view `v` at their positions
     const char *nv;
     int64_t nv_st, nv_sh;
-    int attn_wgs;         // workgroups of the attention grid (the copy workgroups follow)
+    // key rows of the step's tokens before their rotation: the launch rotates each tile in LDS
+    // and writes its block's rows into the arena (instances that rotate keys only)
+    const char *nk;
+    int64_t nk_st, nk_sh;
+    int by_request;       // work items numbered request by request
 };
-
-constexpr int kCopyTokens = 16;  // value rows of 16 packed tokens per copy workgroup
-
-// Copy workgroup `unit`: for each group of 16 of its packed tokens, wave w copies the value
-// rows (every KV head) of tokens 4w ... 4w + 3 into the arena at their positions within their
-// requests (rows past the capacity are not stored), all of a group's loads issued before its
-// first store.
-template <int D>
-Q3T_DEVICE void copy_value_rows(const PrefillParams &p, int unit) {
-    constexpr int CPR = D / 8;  // 16-byte chunks per row
-    constexpr int PER = 8;      // chunks per lane in flight
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int start_l = 0x7fffffff;
-    int64_t slot_l = 0;
-    if (p.B <= 64 && lane < p.B) {
-        start_l = p.cu[lane];
-        slot_l = p.slots ? p.slots[lane] : lane;
-    }
-    const int chunks = p.Hkv * CPR;  // per token
-    for (int group = 0; group < kCopyTokens / 16; ++group) {
-        const int t0 = unit * kCopyTokens + group * 16 + 4 * wave;
-        if (t0 >= p.T) break;
-        // the four tokens' arena row offsets (elements), -1 for no row
-        int64_t row[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int t = t0 + j;
-            row[j] = -1;
-            if (t >= p.T) continue;
-            int start;
-            int64_t slot;
-            if (p.B <= 64) {
-                const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(start_l <= t));
-                const int b = n > 0 ? n - 1 : 0;
-                start = __builtin_amdgcn_readlane(start_l, b);
-                slot = ((int64_t)__builtin_amdgcn_readlane((int)(slot_l >> 32), b) << 32) |
-                       (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)slot_l, b);
-            } else {
-                const int b = request_of(p.cu, p.B, t);
-                start = p.cu[b];
-                slot = p.slots ? p.slots[b] : b;
-            }
-            const int pos = t - start;
-            if (pos >= 0 && pos < p.cap) row[j] = slot * p.v_sb + (int64_t)pos * p.v_st;
-        }
-        for (int f0 = 0; f0 < 4 * chunks; f0 += 64 * PER) {
-            U4 buf[PER];
-            int64_t dst[PER];
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int f = f0 + 64 * i + lane, j = f / chunks, it = f % chunks;
-                const int hh = it / CPR, ch = it % CPR;
-                const int64_t r = j == 0 ? row[0] : j == 1 ? row[1] : j == 2 ? row[2] : j == 3 ? row[3] : -1;
-                dst[i] = r < 0 ? -1 : (r + hh * p.v_sh) * 2 + ch * 16;
-                buf[i] = dst[i] < 0 ? U4{0u, 0u, 0u, 0u}
-                                    : load16(p.nv + ((int64_t)(t0 + j) * p.nv_st + hh * p.nv_sh) * 2 + ch * 16);
-            }
-#pragma unroll
-            for (int i = 0; i < PER; ++i)
-                if (dst[i] >= 0) store16(p.v + dst[i], buf[i]);
-        }
-    }
-}
 
 constexpr float kEmptyP = -1.0e30f;  // finite running maximum before any visible key (masked)
 
@@ -265,39 +215,75 @@ Q3T_DEVICE void mask_values(uint32_t addr, int mdt, float (&mv)[4]) {
     }
 }
 
+// A wave's share of a tile's K or V rows: N loads of 1 KiB, consecutive in LDS.
+template <int N>
+Q3T_DEVICE void load_tile(i32x4_t rs, const uint32_t (&o)[N], uint32_t at, uint32_t base) {
+    static_assert(N == 1 || N == 2 || N == 4, "");
+    if constexpr (N == 4)
+        asm volatile("s_mov_b32 m0, %0\n\t" Q3T_VMEM_SGPR_WAIT "buffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
+                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %5, 0 offen lds\n\t"
+                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds"
+                     :: "s"(base), "v"(o[0] + at), "v"(o[1] + at), "v"(o[2] + at), "v"(o[3] + at), "s"(rs) : "memory", "m0", "scc");
+    else if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %0\n\t" Q3T_VMEM_SGPR_WAIT "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+                     :: "s"(base), "v"(o[0] + at), "v"(o[1] + at), "s"(rs) : "memory", "m0", "scc");
+    else
+        load_to_lds16(rs, o[0] + at, base);
+}
+
+Q3T_DEVICE void lds_write8(uint32_t byte_addr, uint32_t lo, uint32_t hi) {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)byte_addr = u32x2_t{lo, hi};
+}
+
 // MB: bytes per mask element (0: no mask, 2: bf16 / fp16, 4: fp32).  Without a mask the
 // causal rule (and the optional per-request key counts) bounds the key tiles of each query
 // block; with a mask every key tile of the view is scored and the mask alone decides, its
-// tile (64 query rows x 32 keys) staged through the same LDS ring as the keys and values.
-template <int D, int GH, int MB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GH == 1 ? 4 : 3)))
-prefill_attention_kernel(PrefillParams p) {
-    constexpr int NT = 256;                       // threads
-    constexpr int KK = D / 32;                    // MFMA steps over the head dimension
-    constexpr int DB = D / 16;                    // 16-row blocks of O^T
+// tile (the block's query rows x 32 keys) staged through the same LDS ring as the keys and
+// values.  RK: the keys arrive unrotated (the step's own projection rows).  `cu`, `slots` and `nb`
+// lead the arguments: they are preloaded into scalar registers, so a wave asks for its row
+// offsets without waiting for the argument block.
+// SUB: 32-key blocks per tile.  One (three stages of 16 KiB, 168 VGPRs, three workgroups per CU)
+// where the launch fills the card; two (two stages of 32 KiB, the blocks' score chains independent
+// of one another, one maximum, barrier and wait for both) where it does not and the longest
+// block's chain of tiles is the launch: kFewGroups.
+template <int D, int GH, int MB, int SUB, bool RK>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SUB == 2 || GH == 1 ? 2 : 3)))
+prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, PrefillParams p) {
+    constexpr int QPW = 32 / GH;                  // queries per wave
+    constexpr int QB = query_block(GH);           // queries per workgroup
+    constexpr int KK = D / 16;                    // MFMA steps over the head dimension
+    constexpr int DB = D / 32;                    // 32-row blocks of O^T
     constexpr int CPR = D / 8;                    // 16-byte chunks per row
     constexpr int ROW = D * 2;                    // bytes per row
+    constexpr int kTile = kKeys * SUB;            // keys of a tile
+    constexpr int kStages = SUB == 2 ? 2 : 3;     // LDS ring depth: loads run kStages - 1 tiles ahead
     constexpr int KBYTES = kTile * ROW;           // K part of a stage
     constexpr int RB = kTile * MB;                // mask bytes per query row of a tile
-    constexpr int MBYTES = kQBlock * RB;          // mask tile of a stage
+    constexpr int MBYTES = QB * RB;               // mask tile of a stage
     constexpr int SBYTES = 2 * KBYTES + MBYTES;   // stage: K rows, V rows, mask rows
-    constexpr int LPT = 2 * kTile * CPR / NT;     // 16-byte loads per thread per tile
+    constexpr int NL = D / 64 * SUB;              // K (and V) loads per wave and tile
     constexpr int LPR = MB ? RB / 16 : 1;         // lanes per mask row
     constexpr int RPI = 64 / LPR;                 // mask rows per wave load
-    constexpr int LPTM = MB ? 16 / RPI : 0;       // mask loads per wave per tile (16 rows)
-    constexpr int WAIT = LPT + LPTM;              // loads of one tile per thread
-    static_assert(LPT >= 1 && (2 * kTile * CPR) % NT == 0, "a tile is whole loads per thread");
-    static_assert(KBYTES % 1024 == 0, "a wave's load never straddles K and V");
+    constexpr int LPTM = MB ? QPW / RPI : 0;      // mask loads per wave per tile
+    constexpr int WAIT = 2 * NL + LPTM;           // loads of one tile per wave
     __shared__ __attribute__((aligned(1024))) uint8_t ring[kStages * SBYTES];
 
+    const int tid = threadIdx.x, lane = tid & 63;
+    int start = 0, next = 0;
+    int64_t slot_l = lane;
+    if (nb <= 64 && lane < nb) {
+        start = cu[lane];
+        next = cu[lane + 1];
+        if (slots) slot_l = slots[lane];
+    }
+    prefetch_kernargs<24 + sizeof(PrefillParams)>();
     // the wave index through readfirstlane: wave-uniform for the compiler too, so that the
     // per-wave load resources stay in scalar registers
-    if ((int)blockIdx.x >= p.attn_wgs) {  // past the attention grid: value rows to copy
-        if constexpr (MB == 0) copy_value_rows<D>(p, (int)blockIdx.x - p.attn_wgs);
-        return;
-    }
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, c = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hi = lane >> 5, col = lane & 31;
     const int hgroups = p.Hq / GH;
     // Placement: the hardware deals workgroup i to XCD i % 8 and, within an XCD, to its 32 CUs
     // in turn, so CU k of an XCD holds the XCD's workgroups k, k + 32, k + 64 at once (three
@@ -306,7 +292,7 @@ prefill_attention_kernel(PrefillParams p) {
     // Measured on the 16-prompt workload (seed 0): the most loaded CU from 27 to 20 tiles.
     const int wg = [&] {
         const int xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
-        const int rounds = p.attn_wgs / (kXcds * kCusPerXcd);  // complete rounds on every XCD
+        const int rounds = (int)gridDim.x / (kXcds * kCusPerXcd);  // complete rounds on every XCD
         if (j >= rounds * kCusPerXcd) return (int)blockIdx.x;
         const int r = j / kCusPerXcd, pos = j % kCusPerXcd;
         const bool flip = (r & 3) == 1 || (r & 3) == 2;
@@ -315,7 +301,7 @@ prefill_attention_kernel(PrefillParams p) {
     const int hq0 = (wg % hgroups) * GH;  // the workgroup's first query head
     const int h = hq0 / p.group;          // the workgroup's KV head
     const int rest = wg / hgroups;
-    // Work item `rest` of this head group: a (64-query block qb, request b) pair, numbered with
+    // Work item `rest` of this head group: a (query block qb, request b) pair, numbered with
     // the longest blocks first.  Up to 64 requests the numbering is dense: only pairs with
     // rows exist, so the grid's round-robin placement over shader engines sees real work
     // evenly (empty slots in between would pile long blocks onto some engines and stall the
@@ -324,31 +310,42 @@ prefill_attention_kernel(PrefillParams p) {
     // (mbcnt), all wave-uniform, with no memory access beyond the row offsets.
     int b, qb, t0, n, kn;
     int64_t slot;
-    if (p.B <= 64) {
-        int start = 0, rows = 0, klen = 0;
-        int64_t slot_l = 0;  // the request's arena slot, loaded with its rows (no later round trip)
-        if (lane < p.B) {
-            start = p.cu[lane];
-            rows = (start < 0 || start >= p.T) ? 0 : (int)min((int64_t)(p.cu[lane + 1] - start), p.T - start);
+    if (nb <= 64) {
+        int rows = 0, klen = 0;
+        if (lane < nb) {
+            rows = (start < 0 || start >= p.T) ? 0 : (int)min((int64_t)(next - start), p.T - start);
             klen = p.kvl ? p.kvl[lane] : rows;
-            slot_l = p.slots ? p.slots[lane] : lane;
         }
-        const int blocks = rows > 0 ? (rows + kQBlock - 1) / kQBlock : 0;
-        int remaining = rest;
+        const int blocks = rows > 0 ? (rows + QB - 1) / QB : 0;
         qb = -1;
         b = 0;
-        for (int level = p.nqb - 1; level >= 0; --level) {
-            const uint64_t has = __builtin_amdgcn_ballot_w64(blocks > level);
-            const int count = __builtin_popcountll(has);
-            if (remaining < count) {
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0u));
-                const uint64_t pick = __builtin_amdgcn_ballot_w64(blocks > level && (int)rank == remaining);
-                b = __builtin_ctzll(pick);
-                qb = level;
-                break;
+        if (p.by_request) {
+            int before = blocks;  // blocks of requests 0 ... lane, then without the lane's own
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int y = __shfl_up(before, off);
+                if (lane >= off) before += y;
             }
-            remaining -= count;
+            const uint64_t done = __builtin_amdgcn_ballot_w64(before <= rest);  // requests wholly before the item
+            if (~done) {
+                b = __builtin_ctzll(~done);
+                qb = __builtin_amdgcn_readlane(before, b) - 1 - rest;
+            }
+        } else {
+            int remaining = rest;
+            for (int level = p.nqb - 1; level >= 0; --level) {
+                const uint64_t has = __builtin_amdgcn_ballot_w64(blocks > level);
+                const int count = __builtin_popcountll(has);
+                if (remaining < count) {
+                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0u));
+                    const uint64_t pick = __builtin_amdgcn_ballot_w64(blocks > level && (int)rank == remaining);
+                    b = __builtin_ctzll(pick);
+                    qb = level;
+                    break;
+                }
+                remaining -= count;
+            }
         }
         if (qb < 0) return;  // past the last block with rows
         t0 = __builtin_amdgcn_readlane(start, b);
@@ -359,126 +356,154 @@ prefill_attention_kernel(PrefillParams p) {
     } else {
         b = rest % p.B;
         qb = p.nqb - 1 - rest / p.B;  // the longest blocks are dispatched first
-        t0 = p.cu[b];
+        t0 = cu[b];
         if (t0 < 0 || t0 >= p.T) return;
-        n = (int)min((int64_t)(p.cu[b + 1] - t0), p.T - t0);  // rows past the packed tokens do not exist
+        n = (int)min((int64_t)(cu[b + 1] - t0), p.T - t0);  // rows past the packed tokens do not exist
         kn = p.kvl ? p.kvl[b] : n;
-        slot = p.slots ? p.slots[b] : b;
+        slot = slots ? slots[b] : b;
     }
-    const int q0 = qb * kQBlock;
+    const int q0 = qb * QB;
     if (q0 >= n) return;
     // keys 0 ... kv_end-1 are visible to this block; the arena holds at most `cap` of them.
     // Causal: up to the block's last query and the request's key count; masked: every key.
-    const int kv_end = MB ? (int)p.cap : (int)min((int64_t)min(min(n, kn), q0 + kQBlock), p.cap);
+    const int kv_end = MB ? (int)p.cap : (int)min((int64_t)min(min(n, kn), q0 + QB), p.cap);
     const int ntiles = kv_end > 0 ? (kv_end + kTile - 1) / kTile : 0;
-    const int wq0 = q0 + 16 * wave;              // first query of this wave
+    const int wq0 = q0 + QPW * wave;             // first query of this wave
     // keys [0, wave_end) can be visible to the wave; steps reaching past mask_from need the
     // per-key rule (the diagonal or the end of the keys).  A wave whose queries all lie past
     // the request (the tail of its last block) scores nothing: it only loads its share of
     // every tile and joins the barriers.
-    const int wave_end = wq0 >= n ? 0 : MB ? kv_end : min(wq0 + 16, kv_end);
+    const int wave_end = wq0 >= n ? 0 : MB ? kv_end : min(wq0 + QPW, kv_end);
     const int mask_from = MB ? kv_end : min(wq0 + 1, kv_end);
-    const int qpos = wq0 + c;
+    const int qpos = wq0 + col % QPW;
+    const int hq = hq0 + col / QPW;              // the column's query head
     const bool qvalid = qpos < n;
-    const int lim = MB ? kv_end - 1 : min(qpos, kv_end - 1);  // last key visible to this lane's query
+    const int lim = MB ? kv_end - 1 : min(qpos, kv_end - 1);  // last key visible to this lane's column
 
-    // tile loader: load i of a thread fills LDS slot s = i * NT + tid (16 bytes) of a stage:
-    // row s / CPR (K rows first, then V rows), physical chunk s % CPR, holding logical chunk
-    // (physical ^ swizzle(row)) of key tile * kTile + row
-    const char *kbase = p.k + (slot * p.k_sb + h * p.k_sh) * 2;
-    const char *vbase = MB == 0 && p.nv ? p.nv + ((int64_t)t0 * p.nv_st + h * p.nv_sh) * 2
-                                        : p.v + (slot * p.v_sb + h * p.v_sh) * 2;
-    const uint32_t kst = (uint32_t)(p.k_st * 2), vst = (uint32_t)((MB == 0 && p.nv ? p.nv_st : p.v_st) * 2);
+    // tile loader: a wave's loads fill 8 SUB K rows and V rows of a stage; physical chunk pc of row
+    // r holds logical chunk pc ^ swizzle(r).  The resources end with key kv_end - 1: rows past it
+    // read zeros.
+    const bool own_values = MB == 0 && p.nv;
+    const char *kbase = RK ? p.nk + ((int64_t)t0 * p.nk_st + h * p.nk_sh) * 2 : p.k + (slot * p.k_sb + h * p.k_sh) * 2;
+    const char *vbase = own_values ? p.nv + ((int64_t)t0 * p.nv_st + h * p.nv_sh) * 2
+                                   : p.v + (slot * p.v_sb + h * p.v_sh) * 2;
+    const uint32_t kst = (uint32_t)((RK ? p.nk_st : p.k_st) * 2), vst = (uint32_t)((own_values ? p.nv_st : p.v_st) * 2);
     const i32x4_t krs = scalar_rsrc(kbase, kv_end > 0 ? (uint32_t)((kv_end - 1) * kst + D * 2) : 0u);
     const i32x4_t vrs = scalar_rsrc(vbase, kv_end > 0 ? (uint32_t)((kv_end - 1) * vst + D * 2) : 0u);
     // mask rows of the request's queries (rows past its queries read zeros)
     const uint32_t mrow = (uint32_t)(p.m_sq * MB);
     const i32x4_t mrs = scalar_rsrc(MB ? p.mask + b * p.m_sb * MB : kbase,
                                     MB ? (uint32_t)((n - 1) * (int64_t)mrow + p.cap * MB) : 0u);
+    auto v_swizzle = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
     const uint32_t ring_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)ring;
-    uint32_t row_off[LPT];
-    int row_of[LPT];
+    uint32_t koff[NL], voff[NL];
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-        const int s = i * NT + tid, rall = s / CPR, pc = s % CPR;
-        const bool is_v = rall >= kTile;
-        const int r = rall % kTile;
-        const int ch = pc ^ ((is_v ? 2 * r : r) & (CPR - 1));
-        row_of[i] = r;
-        row_off[i] = (uint32_t)r * (is_v ? vst : kst) + ch * 16;
+    for (int i = 0; i < NL; ++i) {
+        const int r = 8 * SUB * wave + i * (64 / CPR) + lane / CPR, pc = lane % CPR;
+        koff[i] = (uint32_t)r * kst + ((pc ^ r) & (CPR - 1)) * 16;
+        voff[i] = (uint32_t)r * vst + (pc ^ v_swizzle(r)) * 16;
     }
+    const uint32_t load_base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ring_base + wave * 8 * SUB * ROW));
     auto issue = [&](int kt, int stage) {
-#pragma unroll
-        for (int i = 0; i < LPT; ++i) {
-            const int first_slot = i * NT + wave * 64;             // wave-uniform
-            const bool is_v = first_slot / CPR >= kTile;
-            const int key0 = kt * kTile;
-            const uint32_t off = row_of[i] < kv_end - key0
-                                     ? row_off[i] + (uint32_t)key0 * (is_v ? vst : kst)
-                                     : 0xfffffff0u;
-            load_to_lds16(is_v ? vrs : krs, off,
-                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(ring_base + stage * SBYTES + first_slot * 16)));
-        }
+        const uint32_t at = load_base + stage * SBYTES;
+        load_tile<NL>(krs, koff, (uint32_t)(kt * kTile) * kst, at);
+        load_tile<NL>(vrs, voff, (uint32_t)(kt * kTile) * vst, at + KBYTES);
         if constexpr (MB > 0) {
-            // the wave's own 16 query rows of the mask tile: load i covers rows RPI i ... + RPI - 1
+            // the wave's own query rows of the mask tile: load i covers rows RPI i ... + RPI - 1
 #pragma unroll
             for (int i = 0; i < LPTM; ++i) {
-                const int r = 16 * wave + i * RPI + lane / LPR;
+                const int r = QPW * wave + i * RPI + lane / LPR;
                 const uint32_t off = q0 + r < n ? (uint32_t)(q0 + r) * mrow + (uint32_t)(kt * RB + (lane % LPR) * 16)
                                                 : 0xfffffff0u;
                 load_to_lds16(mrs, off, (uint32_t)__builtin_amdgcn_readfirstlane(
-                                            (int)(ring_base + stage * SBYTES + 2 * KBYTES + (16 * wave + i * RPI) * RB)));
+                                            (int)(ring_base + stage * SBYTES + 2 * KBYTES + (QPW * wave + i * RPI) * RB)));
             }
         }
     };
 
-    // per-lane LDS read addresses within a stage
-    uint32_t ka[KK], va[DB];
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) ka[kk] = c * ROW + (((4 * kk + g) ^ (c & (CPR - 1))) * 16);
+    // per-lane LDS read addresses within a stage: K row `col`, chunk 2 kk + hi (its XOR with the
+    // row moves only the address's low bits, so step kk is an XOR of the first); V key row
+    // 4 hi + i/4 (i = lane % 16), 4 dims of the 16-lane group's 16 (likewise for dim block db)
+    const uint32_t ka = ring_base + col * ROW + ((hi ^ col) & (CPR - 1)) * 16;
+    uint32_t va;
     {
-        const int r = 4 * g + (c >> 2);  // key row of this lane's transposed read (+16 for keys 16..31)
-        const int sw = (2 * r) & (CPR - 1);
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-            va[db] = KBYTES + r * ROW + (((2 * db + ((c >> 1) & 1)) ^ sw) * 16) + 8 * (c & 1);
+        const int i = lane & 15, r = 4 * hi + (i >> 2), chunk = 2 * ((lane >> 4) & 1) + ((i >> 1) & 1);
+        va = ring_base + KBYTES + r * ROW + (chunk ^ v_swizzle(r)) * 16 + 8 * (i & 1);
     }
 
-    // the first tiles go out before anything else waits on memory
+    // The column's query row as B operands (dims 16 kk + 8 hi ... + 7, zeros past the request) and,
+    // with cos/sin, its RoPE.  Rows are loaded whole (CPR lanes of 16 bytes each), staged in the
+    // wave's 32 rows of the ring past its first stage and read back in operand order: loaded
+    // in operand order they came in 32-byte pieces of 32 rows at once, each line four times over.
+    // The first tile is in flight meanwhile; the block's own value rows, if they go to the arena,
+    // come with the queries.
+    constexpr int RPL = 64 / CPR;                 // rows per load
+    const int lr = lane / CPR, lc = lane % CPR;   // row and chunk of a row load
+    auto token = [&](int i) { return t0 + min(wq0 + i, n - 1); };  // the wave's i-th query's token
+    U4 qrow[32 / RPL], crow[QPW / RPL], srow[QPW / RPL], vrow[QPW / RPL];
 #pragma unroll
-    for (int s = 0; s < kStages - 1; ++s)
-        if (s < ntiles) issue(s, s);
-
-    // the wave's query rows as B operands: Q[query c][8g + 32kk ...], zeros past the request
-    bf16x8_t qB[GH][KK];
-    // with cos/sin: the lane's RoPE rows (its query token, dims 32kk + 8g ... + 7 and the same
-    // dims D/2 further), shared by the GH heads
-    U4 rc1[KK / 2], rc2[KK / 2], rs1[KK / 2], rs2[KK / 2];
+    for (int i = 0; i < 32 / RPL; ++i) {
+        const int r = i * RPL + lr;               // column r: query r % QPW of head r / QPW
+        qrow[i] = load16(p.q + ((int64_t)token(r % QPW) * p.q_st + (hq0 + r / QPW) * p.q_sh) * 2 + lc * 16);
+    }
     if (p.cs) {
-        const int64_t tr = (int64_t)(t0 + (qvalid ? qpos : 0)) * p.cs_st * 2;
 #pragma unroll
-        for (int kk = 0; kk < KK / 2; ++kk) {
-            const int d1 = (32 * kk + 8 * g) * 2, d2 = d1 + D;  // bytes of dims d and d + D/2
-            rc1[kk] = load16(p.cs + tr + d1);
-            rc2[kk] = load16(p.cs + tr + d2);
-            rs1[kk] = load16(p.sn + tr + d1);
-            rs2[kk] = load16(p.sn + tr + d2);
+        for (int i = 0; i < QPW / RPL; ++i) {
+            const int64_t at = (int64_t)token(i * RPL + lr) * p.cs_st * 2 + lc * 16;
+            crow[i] = load16(p.cs + at);
+            srow[i] = load16(p.sn + at);
         }
     }
+    // RK: cos/sin of a tile's keys
+    constexpr int RPT = RK ? 512 / CPR : 1, RKN = RK ? kTile / RPT : 1;  // key rows per pass, passes
+    const int rk_row = tid / (CPR / 2), rk_chunk = tid % (CPR / 2);
+    U4 rkc[RKN][4];
+    auto load_rotation = [&](int kt, int u) {
+        const int key = min(kt * kTile + u * RPT + rk_row, n - 1);
+        const int64_t at = (int64_t)(t0 + key) * p.cs_st * 2 + rk_chunk * 16;
+        rkc[u][0] = load16(p.cs + at);
+        rkc[u][1] = load16(p.cs + at + D);
+        rkc[u][2] = load16(p.sn + at);
+        rkc[u][3] = load16(p.sn + at + D);
+    };
+    // one workgroup per KV head and query block copies the values
+    const bool copy_values = own_values && !RK && hq0 % p.group == 0;
+    if (copy_values) {
 #pragma unroll
-    for (int j = 0; j < GH; ++j) {
-        const char *row = p.q + ((int64_t)(t0 + (qvalid ? qpos : 0)) * p.q_st + (hq0 + j) * p.q_sh) * 2;
+        for (int i = 0; i < QPW / RPL; ++i)
+            vrow[i] = load16(p.nv + ((int64_t)token(i * RPL + lr) * p.nv_st + h * p.nv_sh) * 2 + lc * 16);
+    }
+    if (ntiles > 0) issue(0, 0);
+    const uint32_t stage_row = ring_base + SBYTES + wave * 32 * ROW;  // the wave's staging rows
+    auto stage_rows = [&](auto &rows) {
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(rows) / sizeof(U4)); ++i) {
+            const int r = i * RPL + lr;
+            lds_write16(stage_row + r * ROW + ((lc ^ r) & (CPR - 1)) * 16, rows[i]);
+        }
+    };
+    // chunk 2 kk + hi of staged row r
+    auto staged = [&](int r, int kk) { return lds_read16(stage_row + r * ROW + (((2 * kk + hi) ^ r) & (CPR - 1)) * 16); };
+    bf16x8_t qB[KK];
+    {
         U4 qv[KK];
+        stage_rows(qrow);
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) qv[kk] = load16(row + (32 * kk + 8 * g) * 2);
+        for (int kk = 0; kk < KK; ++kk) qv[kk] = staged(col, kk);
         if (p.cs) {
-            // rotate-half RoPE in registers (bf16-exact; the rotated rows are never stored, so
-            // NaN payloads need no canonical form): the lane's dims 32kk + 8g ... + 7 pair with
-            // the same dims of kk + KK/2, which the lane holds as well
+            // rotate-half RoPE in registers (bf16-exact; the rotated rows are never stored, so NaN
+            // payloads need no canonical form): dims of kk pair with those of kk + KK/2
+            U4 c[KK], t[KK];
+            stage_rows(crow);
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) c[kk] = staged(col % QPW, kk);
+            stage_rows(srow);
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) t[kk] = staged(col % QPW, kk);
 #pragma unroll
             for (int kk = 0; kk < KK / 2; ++kk) {
                 U4 y1, y2;
-                rope8<false>(&qv[kk].x, &qv[kk + KK / 2].x, &rc1[kk].x, &rc2[kk].x, &rs1[kk].x, &rs2[kk].x,
+                rope8<false>(&qv[kk].x, &qv[kk + KK / 2].x, &c[kk].x, &c[kk + KK / 2].x, &t[kk].x, &t[kk + KK / 2].x,
                              &y1.x, &y2.x);
                 qv[kk] = y1;
                 qv[kk + KK / 2] = y2;
@@ -487,139 +512,188 @@ prefill_attention_kernel(PrefillParams p) {
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
             if (!qvalid) qv[kk] = U4{0u, 0u, 0u, 0u};
-            qB[j][kk] = as_bf16x8(qv[kk]);
+            qB[kk] = as_bf16x8(qv[kk]);
         }
     }
-
-    f32x4_t acc[GH][DB];
-    float m[GH], l[GH];  // running maximum (scaled log2 units) and this lane's weight sum
+    if (copy_values) {
 #pragma unroll
-    for (int j = 0; j < GH; ++j) {
-        m[j] = 0.f;
-        l[j] = 0.f;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) acc[j][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < QPW / RPL; ++i) {
+            const int64_t pos = wq0 + i * RPL + lr;
+            if (pos < n && pos < p.cap) store16(p.v + (slot * p.v_sb + h * p.v_sh + pos * p.v_st) * 2 + lc * 16, vrow[i]);
+        }
     }
+    if constexpr (RK) {  // the first tile's, in flight over the barriers
+#pragma unroll
+        for (int u = 0; u < RKN; ++u) load_rotation(0, u);
+    }
+    lds_barrier();  // every wave is done with its staging rows
+    if (kStages == 3 && ntiles > 1) issue(1, 1);
+
+    f32x16_t acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[db] = f32x16_t{};
+    float m = 0.f, l = 0.f;  // running maximum (scaled log2 units) and this lane's weight sum
     bool first = true;
     const float sl = p.scale_log2;
 
-    auto step = [&](int kt, uint32_t sbase) {
+    // Every 32-key block of the tile (one past the wave's keys is masked out: a second instance of
+    // the step for half a tile cost 33 register moves in each).  A block's weights go into the
+    // products while the next block's are computed.
+    auto step = [&](int kt, uint32_t stage) {
+        constexpr int NS = SUB;
+        if (kt * kTile >= wave_end) return;  // past this wave's keys
         const int kb0 = kt * kTile;  // first key of the step
-        if (kb0 >= wave_end) return;  // past this wave's keys
-        const bool masked = kb0 + kTile > mask_from;  // the step reaches past the diagonal or the keys
-        const int rel = lim - kb0;
-        float mk[8];
-        if constexpr (MB > 0) {
-            const uint32_t mrow_lds = sbase + 2 * KBYTES + (16 * wave + c) * RB;
-            float lo[4], hi[4];
-            mask_values<MB>(mrow_lds + 4 * g * MB, p.mdt, lo);
-            mask_values<MB>(mrow_lds + (16 + 4 * g) * MB, p.mdt, hi);
+        const uint32_t so = stage * SBYTES;
+        f32x16_t st[NS];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                mk[i] = lo[i];
-                mk[4 + i] = hi[i];
-            }
-        }
-        bf16x8_t pB[GH];
-#pragma unroll
-        for (int j = 0; j < GH; ++j) {
-            // S^T of head j for keys kb0 + 16kb + (4g..4g+3); a wave issuing products goes
-            // first, the others do their softmax meanwhile
-            f32x4_t st0 = {0.f, 0.f, 0.f, 0.f}, st1 = {0.f, 0.f, 0.f, 0.f};
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                const bf16x8_t a0 = as_bf16x8(lds_read16(sbase + ka[kk]));
-                const bf16x8_t a1 = as_bf16x8(lds_read16(sbase + ka[kk] + 16 * ROW));
-                st0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qB[j][kk], st0, 0, 0, 0);
-                st1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qB[j][kk], st1, 0, 0, 0);
-            }
-            __builtin_amdgcn_s_setprio(0);
-            float x[8] = {st0[0], st0[1], st0[2], st0[3], st1[0], st1[1], st1[2], st1[3]};
-            if constexpr (MB > 0) {  // scores in log2 units with the mask added
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = __builtin_fmaf(x[e], sl, mk[e]);
-            }
-            if (masked) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (4 * g + i > rel) x[i] = -INFINITY;
-                    if (16 + 4 * g + i > rel) x[4 + i] = -INFINITY;
-                }
-            }
-            float mx = x[0];
-#pragma unroll
-            for (int e = 1; e < 8; ++e) mx = __builtin_amdgcn_fmed3f(mx, x[e], __builtin_inff());
-            // the step maximum of a query is the largest of its four lanes' maxima (scaling is
-            // monotonic, so it commutes with the maximum): some query exceeds its running maximum
-            // by more than kRescaleLog2 exactly when some lane's own maximum does, and the
-            // maximum across lanes is needed only to start and to rescale
-            float mt = MB ? mx : mx * sl;
-            if (first || __builtin_amdgcn_ballot_w64(mt > m[j] + kRescaleLog2) != 0) {
-                mt = __builtin_amdgcn_fmed3f(mt, xor16(mt), __builtin_inff());
-                mt = __builtin_amdgcn_fmed3f(mt, xor32(mt), __builtin_inff());
-                if constexpr (MB > 0) mt = fmaxf(mt, kEmptyP);  // a fully masked step keeps m finite
-                if (first) {
-                    m[j] = mt;
-                } else {
-                    const float mn = fmaxf(m[j], mt);
-                    const float alpha = fexp2(m[j] - mn);
-                    m[j] = mn;
-                    l[j] *= alpha;
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) acc[j][db] *= alpha;
-                }
-            }
-            float pv[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pv[e] = MB ? fexp2(x[e] - m[j]) : fexp2(__builtin_fmaf(x[e], sl, -m[j]));
-            l[j] += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
-            const U4 packed = {cvt_pk_bf16(pv[0], pv[1]), cvt_pk_bf16(pv[2], pv[3]),
-                               cvt_pk_bf16(pv[4], pv[5]), cvt_pk_bf16(pv[6], pv[7])};
-            pB[j] = as_bf16x8(packed);
-        }
-        first = false;
-        // O^T += V^T . P^T, one V read for every head
+        for (int u = 0; u < NS; ++u) st[u] = f32x16_t{};
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            const uint2 lo = lds_read_tr16(sbase + va[db]), hi = lds_read_tr16(sbase + va[db] + 16 * ROW);
-            const bf16x8_t av = as_bf16x8(U4{lo.x, lo.y, hi.x, hi.y});
+        for (int kk = 0; kk < KK; ++kk)
 #pragma unroll
-            for (int j = 0; j < GH; ++j)
-                acc[j][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pB[j], acc[j][db], 0, 0, 0);
+            for (int u = 0; u < NS; ++u)
+                st[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(lds_read16((ka ^ (32 * kk)) + so + u * 32 * ROW)), qB[kk], st[u], 0, 0, 0);
+        if constexpr (SUB == 2) {
+            // K fragments three products ahead: left alone, the compiler reads each fragment right in
+            // front of its product and waits a whole LDS latency for every one (one prompt of 2048 43.2 ->
+            // 41.0 us; with one block per tile the registers for it spill)
+            constexpr int MFMA = 0x8, DS_READ = 0x100, AHEAD = 3;
+            __builtin_amdgcn_sched_group_barrier(DS_READ, AHEAD * NS, 0);
+#pragma unroll
+            for (int kk = 0; kk < KK - AHEAD; ++kk) {
+                __builtin_amdgcn_sched_group_barrier(MFMA, NS, 0);
+                __builtin_amdgcn_sched_group_barrier(DS_READ, NS, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(MFMA, AHEAD * NS, 0);
         }
         __builtin_amdgcn_s_setprio(0);
+        float x[16 * NS];
+#pragma unroll
+        for (int e = 0; e < 16 * NS; ++e) x[e] = st[e / 16][e % 16];
+        if constexpr (MB > 0) {  // scores in log2 units with the mask added
+            const uint32_t mrow_lds = ring_base + so + 2 * KBYTES + (QPW * wave + col % QPW) * RB;
+#pragma unroll
+            for (int i = 0; i < 4 * NS; ++i) {
+                float mk[4];
+                mask_values<MB>(mrow_lds + (8 * i + 4 * hi) * MB, p.mdt, mk);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * i + e] = __builtin_fmaf(x[4 * i + e], sl, mk[e]);
+            }
+        }
+        if (kb0 + 32 * NS > mask_from) {  // the step reaches past the diagonal or the keys
+            int rel = lim - kb0 - 4 * hi;
+            asm volatile("" : "+v"(rel));  // keeps the comparisons inside the branch
+#pragma unroll
+            for (int e = 0; e < 16 * NS; ++e)
+                if (8 * (e / 4) + e % 4 > rel) x[e] = -INFINITY;
+        }
+        float mx = x[0];
+#pragma unroll
+        for (int e = 1; e < 16 * NS; ++e) mx = __builtin_amdgcn_fmed3f(mx, x[e], __builtin_inff());
+        // a column's step maximum is the larger of its two lanes' (scaling is monotonic, so it
+        // commutes with the maximum): some column exceeds its running maximum by more than
+        // kRescaleLog2 exactly when some lane's own maximum does, and the maximum across lanes is
+        // needed only to start and to rescale
+        float mt = MB ? mx : mx * sl;
+        if (first || __builtin_amdgcn_ballot_w64(mt > m + kRescaleLog2) != 0) {
+            mt = __builtin_amdgcn_fmed3f(mt, xor32(mt), __builtin_inff());
+            if constexpr (MB > 0) mt = fmaxf(mt, kEmptyP);  // a fully masked step keeps m finite
+            if (first) {
+                m = mt;
+            } else {
+                const float mn = fmaxf(m, mt);
+                const float alpha = fexp2(m - mn);
+                m = mn;
+                l *= alpha;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) acc[db] *= alpha;
+            }
+            first = false;
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * NS; ++u) {
+            float pv[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pv[e] = MB ? fexp2(x[8 * u + e] - m) : fexp2(__builtin_fmaf(x[8 * u + e], sl, -m));
+            l += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+            const bf16x8_t pB = as_bf16x8(U4{cvt_pk_bf16(pv[0], pv[1]), cvt_pk_bf16(pv[2], pv[3]),
+                                             cvt_pk_bf16(pv[4], pv[5]), cvt_pk_bf16(pv[6], pv[7])});
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const uint32_t at = (va ^ (64 * db)) + so + 16 * u * ROW;
+                const uint2 lo = lds_read_tr16(at), up = lds_read_tr16(at + 8 * ROW);
+                acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(U4{lo.x, lo.y, up.x, up.y}), pB, acc[db], 0, 0, 0);
+            }
+        }
     };
-    // one ring position: wait for this tile's loads (later tiles stay in flight), barrier
-    // (every wave is done with the stage the next load overwrites), issue the tile
-    // kStages - 1 ahead into that stage, then the products
+    // RK: a landed tile's keys are rotated in LDS, a thread taking chunks pc and pc + CPR/2 of row
+    // tid / (CPR/2) of every RPT; the block's own rows go to the arena, keys and values
+    auto rotate_keys = [&](int kt, uint32_t stage) {
+#pragma unroll
+        for (int u = 0; u < RKN; ++u) {
+            const int r = u * RPT + rk_row, key = kt * kTile + r;
+            if (key >= kv_end) continue;
+            if (kt > 0) load_rotation(kt, u);
+            const uint32_t row = ring_base + stage * SBYTES + r * ROW;
+            const uint32_t k1 = row + ((rk_chunk ^ r) & (CPR - 1)) * 16, k2 = row + (((rk_chunk + CPR / 2) ^ r) & (CPR - 1)) * 16;
+            const U4 x1 = lds_read16(k1), x2 = lds_read16(k2);
+            U4 y1, y2;
+            rope8(&x1.x, &x2.x, &rkc[u][0].x, &rkc[u][1].x, &rkc[u][2].x, &rkc[u][3].x, &y1.x, &y2.x);
+            lds_write16(k1, y1);
+            lds_write16(k2, y2);
+            if (key >= q0 && hq0 % p.group == 0) {
+                char *ak = const_cast<char *>(p.k) + (slot * p.k_sb + h * p.k_sh + (int64_t)key * p.k_st) * 2 + rk_chunk * 16;
+                char *av = p.v + (slot * p.v_sb + h * p.v_sh + (int64_t)key * p.v_st) * 2 + rk_chunk * 16;
+                store16(ak, y1);
+                store16(ak + D, y2);
+                store16(av, lds_read16(row + KBYTES + (rk_chunk ^ v_swizzle(r)) * 16));
+                store16(av + D, lds_read16(row + KBYTES + ((rk_chunk + CPR / 2) ^ v_swizzle(r)) * 16));
+            }
+        }
+    };
+    // one ring position: wait for this tile's loads (a younger tile stays in flight with three
+    // stages), barrier (every wave is done with the stage the next load overwrites), issue the
+    // tile kStages - 1 ahead into that stage, then the products
     auto ring_step = [&](int kt, int stage) {
-        if (kt + 1 < ntiles) wait_loads<WAIT>();  // the one younger tile stays in flight
+        if (kStages == 3 && kt + 1 < ntiles) wait_loads<WAIT>();
         else wait_loads<0>();
         lds_barrier();
         if (kt + kStages - 1 < ntiles) issue(kt + kStages - 1, (stage + kStages - 1) % kStages);
-        step(kt, ring_base + stage * SBYTES);
+        if constexpr (RK) {
+            rotate_keys(kt, stage);
+            lds_barrier();
+        }
+        step(kt, stage);
     };
-    static_assert(kStages == 3, "the waits above and the unrolled ring below assume three stages");
-    for (int kt = 0; kt < ntiles; kt += kStages) {
-        ring_step(kt, 0);
-        if (kt + 1 < ntiles) ring_step(kt + 1, 1);
-        if (kt + 2 < ntiles) ring_step(kt + 2, 2);
+    if constexpr (RK) {  // one tile, unless a request is longer than the caller said
+        for (int kt = 0; kt < ntiles; ++kt) ring_step(kt, kt % kStages);
+    } else {
+        for (int kt = 0; kt < ntiles; kt += kStages) {
+            ring_step(kt, 0);
+            if (kt + 1 < ntiles) ring_step(kt + 1, 1);
+            if (kStages == 3 && kt + 2 < ntiles) ring_step(kt + 2, kStages - 1);
+        }
     }
 
-    if (!qvalid) return;
-#pragma unroll
-    for (int j = 0; j < GH; ++j) {
-        float lt = l[j] + xor16(l[j]);
-        lt += xor32(lt);
+    // The output rows go through LDS (the wave's 32 rows, swizzled chunks) so that each is stored
+    // whole, CPR lanes of 16 bytes, and not in 16-byte pieces of 32 rows at once.
+    lds_barrier();  // every wave is done with the ring
+    {
+        const float lt = l + xor32(l);
         const float inv = lt > 0.f ? __builtin_amdgcn_rcpf(lt) : 0.f;  // no visible key: zero row
-        char *orow = p.out + ((int64_t)(t0 + qpos) * p.o_st + (hq0 + j) * p.o_sh) * 2;
+        const uint32_t rows = ring_base + wave * 32 * ROW;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            const uint2 v = {cvt_pk_bf16(acc[j][db][0] * inv, acc[j][db][1] * inv),
-                             cvt_pk_bf16(acc[j][db][2] * inv, acc[j][db][3] * inv)};
-            *reinterpret_cast<uint2 *>(orow + (16 * db + 4 * g) * 2) = v;
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                lds_write8(rows + col * ROW + (((4 * db + i) ^ col) & (CPR - 1)) * 16 + 8 * hi,
+                           cvt_pk_bf16(acc[db][4 * i] * inv, acc[db][4 * i + 1] * inv),
+                           cvt_pk_bf16(acc[db][4 * i + 2] * inv, acc[db][4 * i + 3] * inv));
+#pragma unroll
+        for (int i = 0; i < 32 / RPL; ++i) {
+            const int r = i * RPL + lr, pos = wq0 + r % QPW;
+            const U4 v = lds_read16(rows + r * ROW + ((lc ^ r) & (CPR - 1)) * 16);
+            if (pos < n) store16(p.out + ((int64_t)(t0 + pos) * p.o_st + (hq0 + r / QPW) * p.o_sh) * 2 + lc * 16, v);
         }
     }
 }
@@ -628,14 +702,17 @@ prefill_attention_kernel(PrefillParams p) {
 
 using namespace q3t;
 
-extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void *stream) {
+// Validates the arguments and fills the kernel's; `empty`: there is nothing to write.
+static int rope_write_params(const q3t_prefill_rope_write_args *a, PrefillRopeWriteParams &p, bool &empty) {
+    empty = false;
     if (!a) return Q3T_EINVAL;
     if (a->batch < 1 || a->total_tokens < 0 || a->q_heads < 1 || a->kv_heads < 1 ||
         a->capacity < 1 || a->batch > (1 << 20))
         return Q3T_EINVAL;
     if (a->head_dim != 64 && a->head_dim != 128) return Q3T_EUNSUPPORTED;
     if (a->total_tokens > (1 << 30)) return Q3T_EUNSUPPORTED;  // 32-bit token indices
-    if (a->total_tokens == 0) return Q3T_OK;
+    empty = a->total_tokens == 0;
+    if (empty) return Q3T_OK;
     // q_out == NULL: keys and values only (the attention kernel rotates the queries itself)
     const bool with_q = a->q_out != nullptr;
     // value == NULL: keys only (q3t_prefill_attention then copies the values, new_values)
@@ -653,7 +730,6 @@ extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void
                           with_q ? a->q_out : a->key, a->arena_keys, with_v ? a->arena_values : a->key};
     for (const void *q : ptrs)
         if (!aligned(q, 16)) return Q3T_EINVAL;
-    PrefillRopeWriteParams p;
     p.B = (int)a->batch; p.Hq = (int)a->q_heads; p.Hkv = (int)a->kv_heads; p.D = (int)a->head_dim;
     p.T = a->total_tokens; p.capacity = a->capacity; p.cu = a->cu_seqlens;
     p.q = (const char *)a->query; p.k = (const char *)a->key; p.v = (const char *)a->value;
@@ -664,37 +740,83 @@ extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void
     p.ak = (char *)a->arena_keys; p.av = with_v ? (char *)a->arena_values : nullptr;
     p.a_sb = a->a_stride_b; p.a_sh = a->a_stride_h; p.a_st = a->a_stride_t;
     p.slots = a->kv_slots;
+    return Q3T_OK;
+}
+
+static int launch_rope_write(const PrefillRopeWriteParams &p, hipStream_t s) {
     int64_t blocks = (p.T + 3) / 4;  // one token per wave
     if (blocks > 16384) blocks = 16384;
-    hipLaunchKernelGGL(prefill_rope_write_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       (hipStream_t)stream, p);
+    hipLaunchKernelGGL(prefill_rope_write_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p);
     return launch_status();
 }
 
+extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void *stream) {
+    PrefillRopeWriteParams p;
+    bool empty;
+    const int st = rope_write_params(a, p, empty);
+    if (st != Q3T_OK || empty) return st;
+    return launch_rope_write(p, (hipStream_t)stream);
+}
+
+
+// Workgroups from which a launch fills the card (two per CU).  Below, the longest block's chain of
+// tiles bounds it.  us per layer, one / two 32-key blocks per tile: one prompt of 464 18.2 / 14.9 (64
+// workgroups), of 2048 58.2 / 41.0 (256), 8 x 256 under a mask 19.6 / 17.2; 16 prompts of 32..512
+// (664) 25.8 / 31.3, 8 of 1024..2048 92.9 / 97.1.
+constexpr int64_t kFewGroups = 512;
+// Bytes of one KV head's rows of the whole step from which its L2 share no longer holds them.
+constexpr int64_t kL2Rows = 3 << 20;
+
+template <int D, int GH, int SUB>
+static void launch_mask(const PrefillParams &p, const int64_t *slots, dim3 grid, hipStream_t s) {
+    if (!p.mask) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 0, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
+    else if (p.mdt == Q3T_F32) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 4, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
+    else hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 2, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
+}
 
 template <int D, int GH>
-static void launch_prefill(const PrefillParams &p, hipStream_t s) {
+static void launch_prefill(const PrefillParams &p, int64_t max_seqlen, const int64_t *slots, hipStream_t s) {
+    constexpr int QB = query_block(GH);
+    PrefillParams q = p;
+    q.nqb = (int)((max_seqlen + QB - 1) / QB);
     const int64_t hgroups = p.Hq / GH;
-    int64_t wgs = (int64_t)p.B * p.nqb * hgroups;
+    int64_t wgs = (int64_t)p.B * q.nqb * hgroups;
+    // items are numbered densely up to 64 requests: a request of L rows has ceil(L / QB) blocks,
+    // so there are at most (T + (QB - 1) B) / QB of them; rounded up to whole rounds of one
+    // workgroup per CU, which keeps the placement of every item as in the full grid
+    const int64_t items = (p.T + (int64_t)(QB - 1) * p.B) / QB;
     if (p.B <= 64) {
-        // items are numbered densely: a request of L rows has ceil(L / 64) blocks, so there are
-        // at most (T + 63 B) / 64 of them; rounded up to whole rounds of one workgroup per CU,
-        // which keeps the placement of every item as in the full grid
-        const int64_t items = (p.T + (int64_t)(kQBlock - 1) * p.B) / kQBlock;
         const int64_t round = kXcds * kCusPerXcd;
         const int64_t bound = (items * hgroups + round - 1) / round * round;
         if (bound < wgs) wgs = bound;
     }
-    PrefillParams q = p;
-    q.attn_wgs = (int)wgs;
-    if (p.nv) wgs += (p.T + kCopyTokens - 1) / kCopyTokens;
+    // Longest blocks first over all requests ends the launch evenly, but every request's rows are
+    // then in use at once; request by request keeps the rows in use in the XCD's L2.  The latter
+    // where the rows exceed it and the blocks are many against one request's, so that the last
+    // request's chain is a small part of the launch (us per layer, by length / by request: 32
+    // prompts of 500 85.9 / 79.2, 16 of 512 52.5 / 46.4, 8 of 1024..2048 93.7 / 103).
+    q.by_request = p.T * D * 4 > kL2Rows && (int64_t)q.nqb * 8 <= (p.T + QB - 1) / QB;
     const dim3 grid((uint32_t)wgs);
-    if (!p.mask) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 0>), grid, dim3(256), 0, s, q);
-    else if (p.mdt == Q3T_F32) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 4>), grid, dim3(256), 0, s, q);
-    else hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 2>), grid, dim3(256), 0, s, q);
+    if (p.nk) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 0, 2, true>), grid, dim3(256), 0, s, p.cu, slots, p.B, q);
+    else if (wgs <= kFewGroups) launch_mask<D, GH, 2>(q, slots, grid, s);
+    else launch_mask<D, GH, 1>(q, slots, grid, s);
 }
 
-extern "C" int q3t_prefill_attention(const q3t_prefill_args *a, void *stream) {
+static int launch_prefill_sizes(const PrefillParams &p, int64_t head_dim, int64_t max_seqlen, const int64_t *slots, hipStream_t s) {
+    // the query heads of a KV head pair up in one workgroup and share its staged K/V tiles
+    if (p.group % 2 == 0) {
+        if (head_dim == 128) launch_prefill<128, 2>(p, max_seqlen, slots, s);
+        else launch_prefill<64, 2>(p, max_seqlen, slots, s);
+    } else {
+        if (head_dim == 128) launch_prefill<128, 1>(p, max_seqlen, slots, s);
+        else launch_prefill<64, 1>(p, max_seqlen, slots, s);
+    }
+    return launch_status();
+}
+
+// Validates the arguments and fills the kernel's; `empty`: there is nothing to attend.
+static int prefill_params(const q3t_prefill_args *a, PrefillParams &p, bool &empty) {
+    empty = false;
     if (!a) return Q3T_EINVAL;
     if (a->batch < 1 || a->batch > (1 << 20) || a->total_tokens < 0 || a->total_tokens > INT32_MAX ||
         a->max_seqlen < 0 || a->capacity < 1 || a->q_heads < 1 || a->kv_heads < 1 ||
@@ -703,7 +825,8 @@ extern "C" int q3t_prefill_attention(const q3t_prefill_args *a, void *stream) {
     if (a->head_dim != 64 && a->head_dim != 128) return Q3T_EUNSUPPORTED;
     const int64_t G = a->q_heads / a->kv_heads;
     if (G != 1 && G != 2 && G != 4) return Q3T_EUNSUPPORTED;
-    if (a->total_tokens == 0 || a->max_seqlen == 0) return Q3T_OK;
+    empty = a->total_tokens == 0 || a->max_seqlen == 0;
+    if (empty) return Q3T_OK;
     if (!a->cu_seqlens || !a->query || !a->keys || !a->values || !a->out) return Q3T_EINVAL;
     const int64_t st[] = {a->q_stride_t, a->q_stride_h, a->k_stride_b, a->k_stride_h, a->k_stride_t,
                           a->v_stride_b, a->v_stride_h, a->v_stride_t, a->o_stride_t, a->o_stride_h};
@@ -737,12 +860,12 @@ extern "C" int q3t_prefill_attention(const q3t_prefill_args *a, void *stream) {
         const int64_t rows = a->capacity < a->max_seqlen ? a->capacity : a->max_seqlen;
         if (rows * a->nv_stride_t * 2 + a->head_dim * 2 > INT32_MAX) return Q3T_EUNSUPPORTED;
     }
-    PrefillParams p;
+    p = PrefillParams{};
     p.B = (int)a->batch; p.Hq = (int)a->q_heads; p.Hkv = (int)a->kv_heads;
     p.group = (int)G;
-    p.nqb = (int)((a->max_seqlen + kQBlock - 1) / kQBlock);
-    if ((int64_t)p.B * p.nqb * p.Hq + (a->total_tokens + kCopyTokens - 1) / kCopyTokens > INT32_MAX)
-        return Q3T_EUNSUPPORTED;
+    // blocks of 64 queries (128 where a workgroup takes one head)
+    const int64_t blocks = (a->max_seqlen + 63) / 64;
+    if ((int64_t)p.B * blocks * p.Hq > INT32_MAX) return Q3T_EUNSUPPORTED;
     p.scale_log2 = a->scale * kLog2eP;
     p.cu = a->cu_seqlens;
     p.q = (const char *)a->query; p.q_st = a->q_stride_t; p.q_sh = a->q_stride_h;
@@ -759,15 +882,48 @@ extern "C" int q3t_prefill_attention(const q3t_prefill_args *a, void *stream) {
     p.mdt = (int)a->mask_dtype;
     p.m_sb = a->mask_stride_b; p.m_sq = a->mask_stride_q;
     p.nv = (const char *)a->new_values; p.nv_st = a->nv_stride_t; p.nv_sh = a->nv_stride_h;
-    p.attn_wgs = 0;  // set at launch
+    return Q3T_OK;
+}
+
+extern "C" int q3t_prefill_attention(const q3t_prefill_args *a, void *stream) {
+    PrefillParams p;
+    bool empty;
+    const int st = prefill_params(a, p, empty);
+    if (st != Q3T_OK || empty) return st;
+    return launch_prefill_sizes(p, a->head_dim, a->max_seqlen, a->kv_slots, (hipStream_t)stream);
+}
+
+// Whether one launch does the whole layer: the attention's workgroups rotate the keys they read
+// and write their own block's rows, so the keys of a request's earlier blocks are rotated once
+// more in every later one.  Worth it up to kRotateRows rows a request (us per layer, two launches /
+// one: a prompt of 45 rows 10.0 / 8.6, 16 of 64 14.5 / 12.3, 60 of 60 23.7 / 20.3; 3 of 100, two blocks,
+// 12.2 / 13.3).
+constexpr int64_t kRotateRows = 64;
+static bool rotates_keys(const q3t_prefill_rope_write_args *w, const PrefillRopeWriteParams &r,
+                         const q3t_prefill_args *a, const PrefillParams &p) {
+    return a->max_seqlen <= kRotateRows && !a->mask && !a->kv_lens && p.nv && p.cs && !w->q_out && !w->value &&
+           w->arena_keys == a->keys && w->cu_seqlens == a->cu_seqlens && w->kv_slots == a->kv_slots &&
+           w->cos == a->cos && w->sin == a->sin && w->cs_stride_t == a->cs_stride_t && r.B == p.B && r.T == p.T &&
+           r.Hkv == p.Hkv && r.capacity == p.cap && w->head_dim == a->head_dim && r.a_sb == p.k_sb && r.a_sh == p.k_sh &&
+           r.a_st == p.k_st && r.k_st >= 0 && r.k_sh >= 0 && kRotateRows * r.k_st * 2 + a->head_dim * 2 <= INT32_MAX;
+}
+
+extern "C" int q3t_prefill_step(const q3t_prefill_rope_write_args *w, const q3t_prefill_args *a, void *stream) {
+    PrefillRopeWriteParams r;
+    PrefillParams p;
+    bool nothing_to_write, nothing_to_attend;
+    int st = rope_write_params(w, r, nothing_to_write);
+    if (st != Q3T_OK) return st;
+    st = prefill_params(a, p, nothing_to_attend);
+    if (st != Q3T_OK) return st;
     hipStream_t s = (hipStream_t)stream;
-    // the query heads of a KV head pair up in one workgroup and share its staged K/V tiles
-    if (G % 2 == 0) {
-        if (a->head_dim == 128) launch_prefill<128, 2>(p, s);
-        else launch_prefill<64, 2>(p, s);
-    } else {
-        if (a->head_dim == 128) launch_prefill<128, 1>(p, s);
-        else launch_prefill<64, 1>(p, s);
+    if (!nothing_to_write && !nothing_to_attend && rotates_keys(w, r, a, p)) {
+        p.nk = r.k;
+        p.nk_st = r.k_st;
+        p.nk_sh = r.k_sh;
+        return launch_prefill_sizes(p, a->head_dim, a->max_seqlen, a->kv_slots, s);
     }
-    return launch_status();
+    if (!nothing_to_write) st = launch_rope_write(r, s);
+    if (st != Q3T_OK || nothing_to_attend) return st;
+    return launch_prefill_sizes(p, a->head_dim, a->max_seqlen, a->kv_slots, s);
 }

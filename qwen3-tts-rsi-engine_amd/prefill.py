@@ -22,7 +22,7 @@ arena slots, and the attention reads them from there:
 import torch
 
 from . import _lib
-from .attention import prefill_attention
+from .attention import prefill_args, prefill_attention
 
 
 def _check_packed(name, t, tokens, heads, width):
@@ -40,6 +40,15 @@ def prefill_rope_write(query, key, value, cos, sin, cu_seqlens, key_arena, value
     and returns the rotated queries (T, Hq, D), or None with ``rotate_query=False`` (the
     query rows are then not touched).  With ``value=None`` only the keys are written (the
     values are left to ``prefill_attention(new_values=...)``)."""
+    a, q_out, device = _rope_write_args(query, key, value, cos, sin, cu_seqlens, key_arena, value_arena, kv_slots,
+                                        q_out, rotate_query)
+    status = _lib.library().q3t_prefill_rope_write(a, _lib.stream_handle(device))
+    _lib.check(status, 'prefill rope/write')
+    return q_out
+
+
+def _rope_write_args(query, key, value, cos, sin, cu_seqlens, key_arena, value_arena, kv_slots, q_out, rotate_query):
+    """The validated arguments of ``prefill_rope_write``: (arguments, q_out, device)."""
     if query.ndim != 3 or key.ndim != 3:
         raise ValueError('expected packed (tokens, heads, head_dim) rows')
     tokens, q_heads, head_dim = query.shape
@@ -90,9 +99,7 @@ def prefill_rope_write(query, key, value, cos, sin, cu_seqlens, key_arena, value
     a.a_stride_b, a.a_stride_h, a.a_stride_t = key_arena.stride()[:3]
     if kv_slots is not None:
         a.kv_slots = kv_slots.data_ptr()
-    status = _lib.library().q3t_prefill_rope_write(a, _lib.stream_handle(device))
-    _lib.check(status, 'prefill rope/write')
-    return q_out
+    return a, q_out, device
 
 
 def prefill_step(query, key, value, cos, sin, cu_seqlens, max_seqlen, key_arena, value_arena, *,
@@ -100,8 +107,12 @@ def prefill_step(query, key, value, cos, sin, cu_seqlens, max_seqlen, key_arena,
     """One prefill layer over packed prompts: RoPE, arena write, causal GQA.
     Returns the attention output (T, Hq, D).  Two launches: the rotated keys into the arena,
     then attention, which rotates the queries as it loads them, reads the values from
-    ``value`` and copies them into the arena."""
-    prefill_rope_write(query, key, None, cos, sin, cu_seqlens, key_arena, value_arena,
-                       kv_slots=kv_slots, rotate_query=False)
-    return prefill_attention(query, key_arena, value_arena, cu_seqlens, max_seqlen, scale=scale,
-                             kv_slots=kv_slots, out=out, cos=cos, sin=sin, new_values=value)
+    ``value`` and copies them into the arena.  One launch for short prompts (``max_seqlen`` up to
+    64), whose attention rotates the keys as well (q3t_prefill_step)."""
+    write, _, device = _rope_write_args(query, key, None, cos, sin, cu_seqlens, key_arena, value_arena, kv_slots,
+                                        None, False)
+    attend, out, _, _ = prefill_args(query, key_arena, value_arena, cu_seqlens, max_seqlen, scale, kv_slots, out,
+                                     cos, sin, None, None, value)
+    status = _lib.library().q3t_prefill_step(write, attend, _lib.stream_handle(device))
+    _lib.check(status, 'prefill step')
+    return out

@@ -1,0 +1,57 @@
+"""``prefill_step`` over its launch forms: one launch that rotates the keys itself (requests of up
+to 64 rows), tiles of one and two 32-key blocks (launches that fill the card or not), work items
+numbered by length or request by request, and more than 64 requests.
+
+The arena is compared bit for bit with the prologue's (``prefill_rope_write`` of keys and values),
+rows past the requests included; the outputs with float64 attention over the arena (max-abs <=
+2e-2, mean-abs <= 2e-3 for bf16 I/O with fp32 accumulation)."""
+import pytest
+import torch
+
+from tests._util import assert_attention_close, f64
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(pkg, device, lengths, kv_heads, group, head_dim, capacity, seed):
+    gen = torch.Generator(device=device).manual_seed(seed)
+    batch, total = len(lengths), sum(lengths)
+    rows = torch.randn(total, kv_heads * (group + 2), head_dim, generator=gen, device=device, dtype=torch.bfloat16)
+    q, k, v = rows.split([kv_heads * group, kv_heads, kv_heads], dim=1)
+    cu = torch.tensor([0] + lengths).cumsum(0).to(device=device, dtype=torch.int32)
+    cos, sin = pkg.rope_tables(torch.cat([torch.arange(n) for n in lengths]).to(device), head_dim)
+    slots = torch.randperm(batch, generator=torch.Generator().manual_seed(seed)).to(device)
+    arena = torch.randn(2, batch, kv_heads, capacity, head_dim, generator=gen, device=device, dtype=torch.bfloat16)
+    expected = arena.clone()
+    q_rot = pkg.prefill_rope_write(q, k, v, cos, sin, cu, expected[0], expected[1], kv_slots=slots)
+    out = pkg.prefill_step(q, k, v, cos, sin, cu, max(lengths), arena[0], arena[1], kv_slots=slots)
+    torch.cuda.synchronize()
+    assert torch.equal(arena.view(torch.int16), expected.view(torch.int16))
+    want = torch.zeros(out.shape, device=device, dtype=torch.float64)
+    at = 0
+    for b, n in enumerate(lengths):
+        keys, values = (arena[i, slots[b], :, :min(n, capacity)].double().repeat_interleave(group, 0) for i in (0, 1))
+        scores = torch.bmm(q_rot[at:at + n].double().transpose(0, 1).contiguous(), keys.transpose(1, 2).contiguous()) * head_dim ** -0.5
+        hidden = torch.ones(n, keys.shape[1], device=device, dtype=torch.bool).triu(1)
+        weights = scores.masked_fill(hidden, float("-inf")).softmax(-1)
+        want[at:at + n] = torch.bmm(weights, values).transpose(0, 1)
+        at += n
+    assert_attention_close(f64(out), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("group", [1, 2, 4])
+@pytest.mark.parametrize("lengths,capacity", [
+    ([1], 1), ([64], 64), ([1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64], 80), ([64, 20], 40), ([5] * 70, 16)])
+def test_short_requests(pkg, device, lengths, capacity, group, head_dim):
+    _step(pkg, device, lengths, 4, group, head_dim, capacity, 3)
+
+
+@pytest.mark.parametrize("group,head_dim", [(1, 128), (2, 128), (2, 64), (4, 128)])
+@pytest.mark.parametrize("lengths,capacity", [
+    ([65, 128, 129], 129), ([511, 3, 96], 512), ([300, 130], 200),      # few workgroups
+    ([400 + 7 * i for i in range(14)], 512),                            # many, by length
+    ([130 + 4 * i for i in range(40)], 512),                            # many, request by request
+    ([66] * 65, 80)])                                                   # more than 64 requests
+def test_longer_requests(pkg, device, lengths, capacity, group, head_dim):
+    _step(pkg, device, lengths, 8, group, head_dim, capacity, 5)

@@ -221,6 +221,11 @@ int64_t q3t_decode_workspace_bytes(const q3t_decode_args *args);
 
 int q3t_decode_attention(const q3t_decode_args *args, void *stream);
 
+/* q3t_decode_attention with every request at position ctx - 1 (`positions` and `plan` are not
+   read): the operator call over whole key views under a mask (npu_attention.py:11-26), without
+   a launch that fills a vector with one number. */
+int q3t_decode_attention_all_keys(const q3t_decode_args *args, void *stream);
+
 /* The grid q3t_decode_attention would run this call on (Q3T_GRID_CHUNKED, _BALANCED or
    _BUNDLED), from its sizes, `mask`, `splits` and `grid`; Q3T_EUNSUPPORTED when a named grid
    does not take the call, Q3T_EINVAL for malformed sizes.  No counterpart in the reference

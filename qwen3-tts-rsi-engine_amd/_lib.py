@@ -102,6 +102,7 @@ SIGNATURES = {
     "q3t_decode_workspace_bytes": (c_i64, [ctypes.POINTER(DecodeArgs)]),
     "q3t_decode_grid": (ctypes.c_int, [ctypes.POINTER(DecodeArgs)]),
     "q3t_decode_attention": (ctypes.c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
+    "q3t_decode_attention_all_keys": (ctypes.c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
     "q3t_decode_reset_workspace": (ctypes.c_int, [c_vp, c_i64, c_vp]),
     "q3t_decode_plan": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp]),
     "q3t_decode_plan_bytes": (ctypes.c_int64, [c_i64, c_i64, c_i64]),

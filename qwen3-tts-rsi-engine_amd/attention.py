@@ -76,7 +76,8 @@ def _mask_view(mask, batch, query_len, ctx):
     return mask.expand(batch, query_len, ctx)
 
 
-def _run_decode(args: _lib.DecodeArgs, device: torch.device, what: str, no_alloc: bool = False) -> None:
+def _run_decode(args: _lib.DecodeArgs, device: torch.device, what: str, no_alloc: bool = False,
+                all_keys: bool = False) -> None:
     lib = _lib.library()
     with torch.cuda.device(device):
         stream = _lib.stream_handle(device)
@@ -90,7 +91,8 @@ def _run_decode(args: _lib.DecodeArgs, device: torch.device, what: str, no_alloc
                 ws = workspace(device, need, stream)
                 args.workspace = ws.data_ptr()
                 args.workspace_bytes = ws.numel()
-            status = lib.q3t_decode_attention(args, stream)
+            launch = lib.q3t_decode_attention_all_keys if all_keys else lib.q3t_decode_attention
+            status = launch(args, stream)
     _lib.check(status, what)
 
 
@@ -208,6 +210,15 @@ def decode_attention(query, keys, values, positions, *, scale=None, mask=None, k
     overlap in time on one GPU then race).  ``plan``: ``decode_plan(positions, ctx, q_heads,
     kv_heads)`` of these positions, read by the bundled grid (other grids ignore it).
     Returns (B, S, Hq, D)."""
+    if positions.ndim != 1:
+        raise ValueError('positions must be an int64 (batch,) tensor')
+    return _decode_attention(query, keys, values, positions, scale, mask, kv_offsets, out, max_chunks, splits, grid,
+                             no_alloc, plan)
+
+
+def _decode_attention(query, keys, values, positions, scale, mask, kv_offsets=None, out=None, max_chunks=0, splits=0,
+                      grid=None, no_alloc=False, plan=None):
+    """``decode_attention``; ``positions`` None: every request attends all of its keys."""
     if query.ndim != 4 or keys.ndim != 4 or values.shape != keys.shape:
         raise ValueError('expected BSND query and BNSD key/value views')
     batch, qlen, q_heads, head_dim = query.shape
@@ -218,11 +229,11 @@ def decode_attention(query, keys, values, positions, *, scale=None, mask=None, k
         raise ValueError('head_dim mismatch or q_heads not a multiple of kv_heads')
     if query.dtype not in (torch.bfloat16, torch.float32) or keys.dtype != query.dtype or values.dtype != query.dtype:
         raise ValueError('decode attention supports bf16 or fp32 tensors of one dtype')
-    if positions.shape != (batch,) or positions.dtype != torch.int64:
+    if positions is not None and (positions.shape != (batch,) or positions.dtype != torch.int64):
         raise ValueError('positions must be an int64 (batch,) tensor')
     if query.stride(3) != 1 or keys.stride(3) != 1 or values.stride(3) != 1:
         raise ValueError('rows must be unit-stride along head_dim')
-    tensors = [query, keys, values, positions] + ([kv_offsets] if kv_offsets is not None else [])
+    tensors = [query, keys, values] + [t for t in (positions, kv_offsets) if t is not None]
     device = _lib.require_gpu(*tensors)
     if out is None:
         out = torch.empty(batch, qlen, q_heads, head_dim, device=device, dtype=query.dtype)
@@ -243,7 +254,8 @@ def decode_attention(query, keys, values, positions, *, scale=None, mask=None, k
         if kv_offsets.shape != (batch,) or kv_offsets.dtype != torch.int64:
             raise ValueError('kv_offsets must be an int64 (batch,) tensor')
         a.kv_offsets = kv_offsets.data_ptr()
-    a.positions = positions.data_ptr()
+    if positions is not None:
+        a.positions = positions.data_ptr()
     if mask is not None:
         m = _mask_view(mask.to(device), batch, qlen, ctx)
         a.mask = m.data_ptr()
@@ -255,7 +267,7 @@ def decode_attention(query, keys, values, positions, *, scale=None, mask=None, k
     a.splits = int(splits)
     a.grid = _grid_code(grid)
     _set_plan(a, plan, device)
-    _run_decode(a, device, 'decode attention', no_alloc)
+    _run_decode(a, device, 'decode attention', no_alloc, positions is None)
     return out
 
 
@@ -411,15 +423,12 @@ def attention(module, query, key, value, attention_mask, **kwargs):
     mask = attention_mask
     if positions is None:
         if lengths is not None:
-            positions = _length_positions(lengths, device)
-        else:
-            positions = torch.full((batch,), ctx - 1, device=device, dtype=torch.int64)
+            positions = _length_positions(lengths, device)  # else every key: no positions
         if mask is None and 1 < qlen <= 2 and getattr(module, 'is_causal', True):
             # the reference operator's default for several queries: query i sees keys 0 ... i
             mask = torch.ones(qlen, ctx, device=device, dtype=torch.bool).tril()
     if qlen <= 2:
-        out = decode_attention(query.transpose(1, 2), key, value, positions, scale=scale, mask=mask)
-        return out, None
+        return _decode_attention(query.transpose(1, 2), key, value, positions, scale, mask), None
     if kwargs.get('kv_positions') is not None:
         raise ValueError('kv_positions bounds one or two queries per request; for more, pass '
                          'actual_seq_lengths_kv or a mask')

@@ -588,7 +588,7 @@ decode_chunks_kernel(DecodeParams p) {
     const int rest = blockIdx.x / p.Hkv;
     const int c = rest % p.nchunks, b = rest / p.nchunks;
 
-    const int64_t pb = p.pos[b];
+    const int64_t pb = p.pos ? p.pos[b] : p.ctx - 1;
     Work work;
     work.load_rows(p, b, h);
     const int L = (pb >= 0 && pb < p.ctx) ? (int)pb + 1 : 0;
@@ -661,7 +661,7 @@ decode_balanced_kernel(DecodeParams p) {
             const int b = tid * per + e;
             w[e] = 0;
             if (e < per && b < p.B) {
-                const int64_t pb = p.pos[b];
+                const int64_t pb = p.pos ? p.pos[b] : p.ctx - 1;
                 const int L = (pb >= 0 && pb < p.ctx) ? (int)pb + 1 : 0;
                 sm_len[b] = L;
                 w[e] = L > 0 ? L : 1;
@@ -908,7 +908,7 @@ __global__ void __launch_bounds__(kThreads) decode_bundled_kernel(const int32_t 
         int64_t pb[2] = {-1, -1};
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-            if (lane + 64 * e < p.B) pb[e] = p.pos[lane + 64 * e];
+            if (lane + 64 * e < p.B) pb[e] = p.pos ? p.pos[lane + 64 * e] : p.ctx - 1;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int b = lane + 64 * e;
@@ -1573,10 +1573,11 @@ static int dispatch_g(const DecodeParams &p, int g, int sq, bool fused, hipStrea
 
 // Host-side validation and parameter set-up shared by every decode entry point; the device
 // workspace (counter region, then the partial states) starts at `ws`.
-static int decode_params(const q3t_decode_args *a, char *ws, DecodeParams &p) {
+// `all_keys`: every request at position ctx - 1, whatever `positions` holds.
+static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, DecodeParams &p) {
     if (!decode_sizes_ok(a)) return Q3T_EINVAL;
     if (a->kv_heads * a->batch > kMaxCounters) return Q3T_EUNSUPPORTED;
-    if (!a->query || !a->keys || !a->values || !a->positions || !a->out) return Q3T_EINVAL;
+    if (!a->query || !a->keys || !a->values || (!a->positions && !all_keys) || !a->out) return Q3T_EINVAL;
     if (a->dtype != Q3T_BF16 && a->dtype != Q3T_F32) return Q3T_EUNSUPPORTED;
     if (a->head_dim != 64 && a->head_dim != 128) return Q3T_EUNSUPPORTED;
     const int64_t es = a->dtype == Q3T_BF16 ? 2 : 4;
@@ -1625,7 +1626,7 @@ static int decode_params(const q3t_decode_args *a, char *ws, DecodeParams &p) {
     p.k_sb = a->k_stride_b; p.k_sh = a->k_stride_h; p.k_st = a->k_stride_t;
     p.v_sb = a->v_stride_b; p.v_sh = a->v_stride_h; p.v_st = a->v_stride_t;
     p.offs = a->kv_offsets;
-    p.pos = a->positions;
+    p.pos = all_keys ? nullptr : a->positions;
     p.mask = (const char *)a->mask;
     p.m_sb = a->mask_stride_b; p.m_ss = a->mask_stride_s; p.m_st = a->mask_stride_t;
     p.out = (char *)a->out;
@@ -1639,7 +1640,7 @@ static int decode_params(const q3t_decode_args *a, char *ws, DecodeParams &p) {
     p.qnw = nullptr;
     p.knw = nullptr;
     p.eps = a->norm_eps;
-    p.plan = grid == Q3T_GRID_BUNDLED ? a->plan : nullptr;  // read by the bundled grid's two kernels
+    p.plan = grid == Q3T_GRID_BUNDLED && !all_keys ? a->plan : nullptr;  // read by the bundled grid's two kernels
     if (a->q_norm_weight || a->k_norm_weight) {
         if (!fused || !(a->norm_eps >= 0.f)) return Q3T_EINVAL;
         if ((a->q_norm_weight && !aligned(a->q_norm_weight, 16)) ||
@@ -1726,22 +1727,30 @@ extern "C" int q3t_decode_attention_static(const q3t_decode_args *a, void *strea
     char *ws = device_scratch((hipStream_t)stream);
     if (!ws) return (int)hipErrorInvalidDevicePointer;
     DecodeParams p;
-    const int st = decode_params(a, ws, p);
+    const int st = decode_params(a, ws, false, p);
     if (st != Q3T_OK) return st;
     return decode_launch(a, p, stream);
 }
 
-extern "C" int q3t_decode_attention(const q3t_decode_args *a, void *stream) {
+static int decode_with_workspace(const q3t_decode_args *a, bool all_keys, void *stream) {
     if (!a) return Q3T_EINVAL;
     if (!decode_sizes_ok(a)) return Q3T_EINVAL;
     if (a->batch == 0) return Q3T_OK;
     DecodeParams p;
-    const int st = decode_params(a, (char *)a->workspace, p);
+    const int st = decode_params(a, (char *)a->workspace, all_keys, p);
     if (st != Q3T_OK) return st;
     const int64_t need = q3t_decode_workspace_bytes(a);
     if (need > 0 && (!a->workspace || a->workspace_bytes < need || !aligned(a->workspace, 16)))
         return Q3T_EWORKSPACE;
     return decode_launch(a, p, stream);
+}
+
+extern "C" int q3t_decode_attention(const q3t_decode_args *a, void *stream) {
+    return decode_with_workspace(a, false, stream);
+}
+
+extern "C" int q3t_decode_attention_all_keys(const q3t_decode_args *a, void *stream) {
+    return decode_with_workspace(a, true, stream);
 }
 
 static bool plan_shape_ok(int64_t batch, int64_t ctx, int64_t q_heads, int64_t kv_heads) {

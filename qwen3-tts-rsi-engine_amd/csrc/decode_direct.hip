@@ -140,7 +140,7 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
                  "s_load_dwordx4 %[d], %[ka], 0xc8\n\ts_load_dwordx2 %[e], %[ka], 0xd8\n\ts_waitcnt lgkmcnt(0)"
                  : [pb] "=&s"(pb), [a] "=&s"(block.a), [b] "=&s"(block.b), [c] "=&s"(block.c), [d] "=&s"(block.d),
                    [e] "=&s"(block.e)
-                 : [pa] "s"(pos + b), [ka] "s"(__builtin_amdgcn_kernarg_segment_ptr())
+                 : [pa] "s"(pos ? (uint64_t)(uintptr_t)(pos + b) : (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr()), [ka] "s"(__builtin_amdgcn_kernarg_segment_ptr())
                  : "memory");
     struct Packed { uint32_t w[54]; } words;
 #pragma unroll
@@ -154,7 +154,8 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
     words.w[53] = (uint32_t)(block.e >> 32);
     const DirectParams p = __builtin_bit_cast(DirectParams, words);
 
-    const int L = (int64_t)pb >= 0 && (int64_t)pb < p.ctx ? (int)pb + 1 : 0;
+    // without positions every request attends all of its keys
+    const int L = !pos ? p.ctx : (int64_t)pb >= 0 && (int64_t)pb < p.ctx ? (int)pb + 1 : 0;
     char *out = p.out + (b * p.o_sb + h * G * p.o_sh);
     if (L == 0) {  // no valid position: attends nothing, zero rows
         for (int t = tid; t < R * 128; t += W * 64) {

@@ -152,3 +152,21 @@ def test_step_in_a_graph_follows_rewritten_positions(pkg, device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, expected) and torch.equal(keys, keys2) and torch.equal(values, values2)
+
+
+@pytest.mark.parametrize("batch,capacity,dtype,head_dim", [
+    (6, 300, torch.bfloat16, 128), (64, 1024, torch.bfloat16, 128), (4, 2100, torch.bfloat16, 128),
+    (5, 200, torch.float32, 128), (5, 200, torch.bfloat16, 64)])
+def test_the_operator_call_attends_every_key_on_each_grid(pkg, device, batch, capacity, dtype, head_dim):
+    """``attention`` without positions: the launch that reads no position vector, bit for bit the
+    one given the last position of every request."""
+    from types import SimpleNamespace
+    module = SimpleNamespace(training=False, is_causal=True, sliding_window=None)
+    gen = torch.Generator(device=device).manual_seed(capacity)
+    query = torch.randn(batch, 16, 1, head_dim, generator=gen, device=device, dtype=dtype)
+    keys, values = (torch.randn(batch, 8, capacity, head_dim, generator=gen, device=device, dtype=dtype) for _ in range(2))
+    seen = torch.rand(batch, 1, 1, capacity, generator=gen, device=device) < 0.7
+    last = torch.full((batch,), capacity - 1, device=device, dtype=torch.int64)
+    for mask in (seen, None):
+        out, _ = pkg.attention(module, query, keys, values, mask)
+        assert torch.equal(out, pkg.decode_attention(query.transpose(1, 2), keys, values, last, mask=mask))

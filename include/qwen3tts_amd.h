@@ -80,6 +80,15 @@ int q3t_copy_strided(void *dst, const void *src, int64_t elem_size, int ndim,
                      const int64_t *sizes, const int64_t *dst_strides,
                      const int64_t *src_strides, void *stream);
 
+/*
+ * A larger copy of a contiguous arena of planes * slots * heads blocks: each block of dst
+ * (new_bytes) gets the old block's old_bytes and zeros after them; blocks of slots `used` and
+ * past it get zeros.  Q3T_EUNSUPPORTED unless blocks and pointers are 16-byte multiples.
+ * Replaces: ensure_capacity's allocation and copy (continuous.py:353-363).
+ */
+int q3t_grow_arena(void *dst, const void *src, int64_t planes, int64_t slots, int64_t used, int64_t heads,
+                   int64_t old_bytes, int64_t new_bytes, void *stream);
+
 /* Plain contiguous byte copy: the calibration kernel for the HBM byte counters (a copy of
    known size).  No counterpart in the reference; slot moves go through q3t_copy_strided. */
 int q3t_copy_bytes(void *dst, const void *src, int64_t nbytes, void *stream);

@@ -95,6 +95,7 @@ SIGNATURES = {
                                     c_i64, I64x3, I64x3, I64x3, c_i64, c_vp]),
     "q3t_copy_strided": (ctypes.c_int, [c_vp, c_vp, c_i64, ctypes.c_int, ctypes.POINTER(c_i64),
                                         ctypes.POINTER(c_i64), ctypes.POINTER(c_i64), c_vp]),
+    "q3t_grow_arena": (ctypes.c_int, [c_vp, c_vp] + [c_i64] * 6 + [c_vp]),
     "q3t_copy_bytes": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp]),
     "q3t_rotary": (ctypes.c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_vp]),
     "q3t_rope_tables": (ctypes.c_int, [c_vp, c_i64, c_vp, c_i64, ctypes.c_float, c_i64, c_vp,

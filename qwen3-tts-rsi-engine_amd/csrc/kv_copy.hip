@@ -4,11 +4,12 @@
 //                   (reference: continuous.py:152-166, kv_triton_ascend.py:24-64,
 //                    predictor.py:19-24).
 // q3t_copy_strided - up-to-5-D strided copy used for the packed prefix copy, slot
-//                   compaction and arena regrowth (packed_kv.py:6-31,
-//                   continuous.py:118-128, 353-363).
+//                   compaction (packed_kv.py:6-31, continuous.py:118-128).
+// q3t_grow_arena  - a larger arena from a smaller one, copied rows and zeros in one pass
+//                   (continuous.py:353-363).
 // q3t_copy_bytes  - contiguous copy; also the calibration kernel for HBM counters.
 //
-// All three are HBM-bound byte moves: one work item moves one 16-byte vector when the
+// All are HBM-bound byte moves: one work item moves one 16-byte vector when the
 // row, pointers and strides allow it, else the widest power-of-two unit that divides them.
 #include "q3t_common.hpp"
 
@@ -78,6 +79,39 @@ __global__ void __launch_bounds__(256) copy_strided_kernel(CopyParams p) {
         }
         *reinterpret_cast<T *>(p.dst + doff) = *reinterpret_cast<const T *>(p.src + soff);
     }
+}
+
+constexpr int kRunVectors = 4;                    // 16-byte vectors in flight per thread
+constexpr int kRunChunk = 256 * kRunVectors;      // vectors of a workgroup
+
+// A larger arena: block (plane, slot, head) of `dst`, new_vectors long, gets the old block's
+// old_vectors and zeros after them; slots from `used` on get zeros.  One pass that writes every
+// byte of the new arena once (zero-filling it first and copying over it wrote the copied half
+// twice); rows are read and written once and far exceed the caches, so both sides carry the
+// non-temporal policy.  32 slots x 512 rows -> 1024, 28 layers (1.9 GB read, 3.8 GB written):
+// ~1310 us as fill and copy, 1004 us (5.6 TB/s).
+struct GrowParams {
+    char *dst;
+    const char *src;
+    uint32_t chunks, old_vectors, new_vectors;    // chunks per new block
+    uint32_t heads, slots, used;
+};
+__global__ void __launch_bounds__(256) grow_blocks_kernel(GrowParams p) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    const uint32_t block = blockIdx.x / p.chunks, chunk = blockIdx.x % p.chunks;
+    const bool copies = (block / p.heads) % p.slots < p.used;
+    const uint32_t first = chunk * kRunChunk + threadIdx.x;
+    const u32x4_t *src = reinterpret_cast<const u32x4_t *>(p.src) + (uint64_t)block * p.old_vectors;
+    u32x4_t *dst = reinterpret_cast<u32x4_t *>(p.dst) + (uint64_t)block * p.new_vectors;
+    u32x4_t v[kRunVectors];
+#pragma unroll
+    for (int i = 0; i < kRunVectors; ++i) {
+        v[i] = u32x4_t{0u, 0u, 0u, 0u};
+        if (copies && first + 256 * i < p.old_vectors) v[i] = __builtin_nontemporal_load(src + first + 256 * i);
+    }
+#pragma unroll
+    for (int i = 0; i < kRunVectors; ++i)
+        if (first + 256 * i < p.new_vectors) __builtin_nontemporal_store(v[i], dst + first + 256 * i);
 }
 
 static int pick_vec(int64_t row_bytes, int64_t esize, std::initializer_list<int64_t> byte_strides,
@@ -226,4 +260,21 @@ extern "C" int q3t_copy_bytes(void *dst, const void *src, int64_t nbytes, void *
     }
     int64_t one = 1;
     return q3t_copy_strided(dst, src, 1, 1, &nbytes, &one, &one, stream);
+}
+
+extern "C" int q3t_grow_arena(void *dst, const void *src, int64_t planes, int64_t slots, int64_t used, int64_t heads,
+                              int64_t old_bytes, int64_t new_bytes, void *stream) {
+    if (!dst || !src || planes < 1 || slots < 1 || used < 0 || used > slots || heads < 1 || old_bytes < 0 ||
+        new_bytes < old_bytes || new_bytes < 1)
+        return Q3T_EINVAL;
+    if (old_bytes % 16 || new_bytes % 16 || !aligned(dst, 16) || !aligned(src, 16)) return Q3T_EUNSUPPORTED;
+    const int64_t limit = INT32_MAX, vectors = new_bytes / 16, chunks = (vectors + kRunChunk - 1) / kRunChunk;
+    if (planes > limit / slots || planes * slots > limit / heads || vectors > limit ||
+        planes * slots * heads > limit / chunks)
+        return Q3T_EUNSUPPORTED;
+    const GrowParams p = {(char *)dst, (const char *)src, (uint32_t)chunks, (uint32_t)(old_bytes / 16), (uint32_t)vectors,
+                          (uint32_t)heads, (uint32_t)slots, (uint32_t)used};
+    hipLaunchKernelGGL(grow_blocks_kernel, dim3((uint32_t)(planes * slots * heads * chunks)), dim3(256), 0,
+                       (hipStream_t)stream, p);
+    return launch_status();
 }

@@ -55,3 +55,23 @@ def copy_rows(dst: torch.Tensor, src: torch.Tensor) -> None:
     status = _lib.library().q3t_copy_strided(dst.data_ptr(), src.data_ptr(), dst.element_size(),
                                              n, sizes, ds, ss, _lib.stream_handle(device))
     _lib.check(status, "copy_rows")
+
+
+def grow_blocks(dst: torch.Tensor, src: torch.Tensor, used: int) -> None:
+    """dst (planes, slots, heads, new, width) <- src (planes, slots, heads, old, width), old <= new:
+    the rows of slots below ``used``, then zeros; every element of dst is written.  Both
+    contiguous, and rows as the kernel takes them (``can_grow_blocks``)."""
+    device = _lib.require_gpu(dst, src)
+    planes, slots, heads, rows, width = dst.shape
+    size = dst.element_size() * width
+    status = _lib.library().q3t_grow_arena(dst.data_ptr(), src.data_ptr(), planes, slots, used, heads,
+                                           src.shape[3] * size, rows * size, _lib.stream_handle(device))
+    _lib.check(status, "grow_blocks")
+
+
+def can_grow_blocks(dst: torch.Tensor, src: torch.Tensor) -> bool:
+    size = dst.element_size() * dst.shape[-1]
+    return (dst.is_cuda and dst.numel() > 0 and src.numel() > 0 and dst.dtype == src.dtype and dst.is_contiguous()
+            and src.is_contiguous() and dst.data_ptr() % 16 == 0 and src.data_ptr() % 16 == 0
+            and (src.shape[-2] * size) % 16 == 0 and (dst.shape[-2] * size) % 16 == 0
+            and dst.numel() * dst.element_size() // 16 < 1 << 31)

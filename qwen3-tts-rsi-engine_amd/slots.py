@@ -14,7 +14,7 @@ from transformers.cache_utils import Cache
 
 from . import kv_write
 from .attention import PLAN_MAX_BATCH, decode_grid_for, decode_plan, plan_shape
-from .packed_kv import copy_packed_prefix, copy_rows
+from .packed_kv import can_grow_blocks, copy_packed_prefix, copy_rows, grow_blocks
 
 
 def _attention_heads(reference):
@@ -37,6 +37,10 @@ class SlotArena:
 
     def __init__(self, reference, slots, capacity, native_kv_update=False, triton_kv_update=False,
                  packed_kv=False):
+        self._create(torch.zeros, reference, slots, capacity, native_kv_update, triton_kv_update, packed_kv)
+
+    def _create(self, fill, reference, slots, capacity, native_kv_update, triton_kv_update, packed_kv):
+        """``fill``: torch.zeros, or torch.empty for an arena whose every row is written next."""
         self.reference = reference
         self.slots = slots
         self.capacity = capacity
@@ -49,13 +53,12 @@ class SlotArena:
         self.packed = None
         if packed_kv:
             layers = len(reference.layers)
-            self.packed = torch.zeros((layers * 2, *shape), device=weight.device, dtype=weight.dtype)
+            self.packed = fill((layers * 2, *shape), device=weight.device, dtype=weight.dtype)
             self.keys = list(self.packed[:layers].unbind(0))
             self.values = list(self.packed[layers:].unbind(0))
         else:
-            self.keys = [torch.zeros(shape, device=weight.device, dtype=weight.dtype)
-                         for _ in reference.layers]
-            self.values = [torch.zeros_like(key) for key in self.keys]
+            self.keys = [fill(shape, device=weight.device, dtype=weight.dtype) for _ in reference.layers]
+            self.values = [fill(shape, device=weight.device, dtype=weight.dtype) for _ in reference.layers]
 
     def load(self, slot, cache, row=0, length=None):
         """Copy the first ``length`` positions of one prefill cache row into ``slot``."""
@@ -109,9 +112,20 @@ def grow_arena(old: SlotArena, required: int, active: int | None = None) -> Slot
     if required < old.capacity:
         return old
     capacity = max(old.capacity * 2, 1 << int(required).bit_length())
-    new = SlotArena(old.reference, old.slots, capacity, old.native_kv_update, old.triton_kv_update,
-                    packed_kv=old.packed_kv)
     used = old.slots if active is None else max(0, min(int(active), old.slots))
+    sizes = (old.reference, old.slots, capacity, old.native_kv_update, old.triton_kv_update, old.packed_kv)
+    if used > 0:
+        # one pass over the new arena: copied rows and zeros, each byte written once
+        new = SlotArena.__new__(SlotArena)
+        new._create(torch.empty, *sizes)
+        pairs = ([(new.packed, old.packed)] if new.packed is not None
+                 else [(target[None], source[None]) for target, source in zip(new.planes(), old.planes())])
+        if all(can_grow_blocks(target, source) for target, source in pairs):
+            for target, source in pairs:
+                grow_blocks(target, source, used)
+            return new
+        del new, pairs
+    new = SlotArena(*sizes)
     if used == 0:
         return new
     if new.packed is not None:

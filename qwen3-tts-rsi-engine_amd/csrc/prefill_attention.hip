@@ -165,7 +165,7 @@ struct PrefillParams {
     const char *q;
     int64_t q_st, q_sh;
     const char *k;
-    char *v;  // written only with nv (the copy workgroups)
+    char *v;  // written only with nv
     int64_t k_sb, k_sh, k_st, v_sb, v_sh, v_st;
     int64_t cap;
     const int64_t *slots;

@@ -141,7 +141,10 @@ int q3t_rope_tables(const int64_t *positions, int64_t n, const float *inv_freq, 
  *     head cut into equal shares, one per workgroup; the default otherwise for ctx >= 2048.
  *   - chunked: each request's keys cut into chunks of 64-key blocks (at most `max_chunks`
  *     per request), one workgroup per (request, chunk, KV head); the default otherwise (the
- *     code predictor's 16-row caches, short arenas, few requests).
+ *     code predictor's 16-row caches, short arenas, few requests).  With max_chunks <= 0 and
+ *     splits == 0, bf16 rows of 128 below 2048 keys, and unfused fp32 rows or bf16 rows of 64
+ *     whose planes are short and few, run unsplit: one workgroup per (request, KV head); over
+ *     bf16 rows of 128 it reads no key behind the last one that a mask shows.
  * A request covered by several workgroups (balanced, chunked) merges their partial softmax
  * states through `workspace`; the last workgroup to finish writes the output.
  *
@@ -189,7 +192,8 @@ typedef struct q3t_decode_args {
     /* workspace (chunked and balanced grids): a fixed 256 KiB counter region
        (kv_heads * batch <= 65536), then the partial states of split requests; zero-filled
        before first use, its counters left zeroed by every launch.  Launches that overlap in
-       time must not share one.  The bundled grid uses none (may be NULL). */
+       time must not share one.  The bundled grid uses none (may be NULL); calls that
+       run unsplit on the chunked grid leave theirs untouched. */
     void *workspace;
     int64_t workspace_bytes;
     int64_t max_chunks;      /* chunked grid: chunks per request and KV head, <= 1024; <= 0:

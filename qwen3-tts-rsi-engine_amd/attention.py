@@ -204,7 +204,7 @@ def decode_attention(query, keys, values, positions, *, scale=None, mask=None, k
     stride; one query token, head_dim 128, up to 128 requests), 'balanced'
     (equal shares of each head's keys over ``splits`` workgroups per head, 0: 256 in all),
     'chunked' (chunks of 64-key blocks per request, at most ``max_chunks``, 0: enough for
-    ~512 workgroups) or None for the library's choice, in which ``splits`` > 0 / < 0 still
+    ~512 workgroups, or one workgroup per request and head where that is faster) or None for the library's choice, in which ``splits`` > 0 / < 0 still
     selects balanced / chunked.  ``no_alloc`` runs the library's allocation-free entry point, which keeps
     its split states in a fixed per-GPU device array instead of a workspace (calls that
     overlap in time on one GPU then race).  ``plan``: ``decode_plan(positions, ctx, q_heads,

@@ -22,7 +22,8 @@
 //   * chunked (small caches, the code predictor, short arenas): one workgroup per (request,
 //     chunk of 64-key blocks, KV head), whose rows are requested together with its position.
 //     bf16 calls over rows of 128 that set no chunk count run unsplit instead, one workgroup per
-//     (request, KV head) (decode_direct.hip; direct_ok).
+//     (request, KV head) (decode_direct.hip; direct_ok), and so do unfused fp32 calls and bf16
+//     rows of 64 over short planes (decode_whole.hip; whole_ok).
 // For these two:
 //   * lanes: 16 bytes of one key row per lane (LPK lanes per key); a pass of the workgroup
 //     reads 4 KiB of K and 4 KiB of V, all passes of a block are issued before any math;

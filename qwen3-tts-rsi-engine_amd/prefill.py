@@ -17,7 +17,7 @@ arena slots, and the attention reads them from there:
 * ``prefill_step`` - one layer: the key prologue, then attention over the raw queries with
   their RoPE applied in the attention kernel (no rotated copy of the queries is written),
   reading the values from the projection's rows while the same launch copies them into the
-  arena.
+  arena; one launch for both up to 64 rows a request (kernel ``q3t_prefill_step``).
 """
 import torch
 

@@ -22,8 +22,8 @@
 //   * chunked (small caches, the code predictor, short arenas): one workgroup per (request,
 //     chunk of 64-key blocks, KV head), whose rows are requested together with its position.
 //     bf16 calls over rows of 128 that set no chunk count run unsplit instead, one workgroup per
-//     (request, KV head) (decode_direct.hip; direct_ok), and so do unfused fp32 calls and bf16
-//     rows of 64 over short planes (decode_whole.hip; whole_ok).
+//     (request, KV head) (decode_direct.hip; direct_ok), and so do unfused bf16 calls over rows of
+//     64 and short planes (decode_whole.hip; whole_ok).
 // For these two:
 //   * lanes: 16 bytes of one key row per lane (LPK lanes per key); a pass of the workgroup
 //     reads 4 KiB of K and 4 KiB of V, all passes of a block are issued before any math;
@@ -974,12 +974,13 @@ static bool direct_ok(const q3t_decode_args *a) {
     return true;
 }
 // Whether a call on the chunked grid that would split its requests runs one workgroup per (request,
-// KV head) instead (decode_whole.hip): fp32 rows, or bf16 rows of 64.
+// KV head) instead (decode_whole.hip): bf16 rows of 64.  Not fp32: the launch was 8% of an fp32 step
+// faster, but its error against float64, in other order of the same sums, 1-3% above the split one's.
 static bool whole_ok(const q3t_decode_args *a) {
     const int64_t G = a->q_heads / a->kv_heads;
-    return (a->dtype == Q3T_F32 || a->head_dim == 64) && !a->fused && (G == 1 || G == 2 || G == 4) &&
+    return a->dtype == Q3T_BF16 && a->head_dim == 64 && !a->fused && (G == 1 || G == 2 || G == 4) &&
            (a->query_len == 1 || a->query_len == 2) && G * a->query_len <= 4 && a->ctx > kWholeMinCtx &&
-           a->ctx * a->head_dim * (a->dtype == Q3T_F32 ? 4 : 2) <= kWholeMaxPlane && a->splits == 0 &&
+           a->ctx * a->head_dim * 2 <= kWholeMaxPlane && a->splits == 0 &&
            a->max_chunks <= 0 && a->batch * a->kv_heads <= kWholeMaxPairs;
 }
 static int decode_grid(const q3t_decode_args *a) {
@@ -1240,7 +1241,7 @@ static int decode_launch(const q3t_decode_args *a, const DecodeParams &p, void *
         return launch_status();
     }
     if (decode_grid(a) == Q3T_GRID_CHUNKED && whole_ok(a)) {
-        whole_launch(p, a->dtype == Q3T_F32, (int)a->head_dim, g, sq, s);
+        whole_launch(p, g, sq, s);
         return launch_status();
     }
     int st;

@@ -53,7 +53,7 @@ void direct_launch(const DecodeParams &p, int group, int tokens, bool fused, hip
 constexpr int kWholeMinCtx = 64;             // one block of keys needs no more waves
 constexpr int kWholeMaxPlane = 256 << 10;    // bytes of a head's key rows
 constexpr int kWholeMaxPairs = 256;          // one workgroup per CU
-void whole_launch(const DecodeParams &p, bool f32, int head_dim, int group, int tokens, hipStream_t s);
+void whole_launch(const DecodeParams &p, int group, int tokens, hipStream_t s);
 
 // 4 bytes per lane from global memory into LDS at lds_base + 4 * lane (the mask words of a
 // stage's rows); offsets past the resource's range write zeros.

@@ -14,10 +14,11 @@
 //     LDS (16 bytes per lane, rows of 16-byte chunks XOR-swizzled as in the bundled grid), two
 //     stages of its own in flight, with no barrier in the stream;
 //   * S^T = K . Q^T and O^T += V^T . P^T run on bf16 MFMA tiles whose 16 columns are mostly
-//     empty, so the weights keep their precision for free: columns 0 ... R-1 carry the weights
-//     rounded to bf16, columns R ... 2R-1 (the same queries again) the rounding remainders, and
-//     the two are added at the end.  The products then see 16 significant bits of each weight
-//     (relative error 2^-17) at the cost of one column's MFMA;
+//     empty, so the weights keep all 24 bits of their float32: columns 0 ... R-1 carry the weights
+//     rounded to bf16, columns R ... 2R-1 (the same queries again) the remainders rounded to bf16
+//     and columns 2R ... 3R-1 what is left of those, which is exact; the three are added at the
+//     end.  Eight query rows (R = 8) leave no columns for the third part: a second product of the
+//     same V fragments adds it;
 // A wave issues one instruction every four cycles here (one wave per SIMD), so the instructions
 // on the chain count as much as its round trips: arguments straight into scalar registers,
 // 32-bit row offsets, resources that end at the last key instead of per-lane bounds, four loads
@@ -75,9 +76,11 @@ struct DirectLds {
 Q3T_DEVICE uint32_t lds_read4(uint32_t byte_addr) {
     return *(__attribute__((address_space(3))) const uint32_t *)(uintptr_t)byte_addr;
 }
-// The value of the lane R above within a 16-lane row (lanes past the row: 0).
-template <int R>
-Q3T_DEVICE float from_above(float x) { return dpp<0x100 + R>(x); }
+// What rounding to bf16 left of two floats (exact).
+Q3T_DEVICE void bf16_rest(float &a, float &b, uint32_t rounded) {
+    a -= bf16_lo(rounded);
+    b -= bf16_hi(rounded);
+}
 
 // Four 1 KiB loads of a stage's K or V rows (rows 4i + lane / 16, chunk lane % 16) into LDS.  The
 // instruction's offset moves the memory and the LDS address alike, so load i's voffset is 1024 i
@@ -119,7 +122,10 @@ __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))
 decode_direct_kernel(const int64_t *pos, DirectParams) {
     constexpr bool FUSED = FUSE > 0, NORM = FUSE > 1;
     constexpr int R = G * SQ;               // query rows
-    static_assert(2 * R <= 16, "each query row takes two of the 16 columns");
+    // columns of a query row: its weights in two or three bf16 parts
+    constexpr bool THIRD = 3 * R <= 16;
+    constexpr int COLS = (THIRD ? 3 : 2) * R;
+    static_assert(2 * R <= 16, "each query row takes two of the 16 columns at least");
     // rows in LDS: queries, then (fused) cos, sin, new keys and new values of each token, and
     // the norm weights
     constexpr int COS = R, SIN = R + SQ, NEWK = R + 2 * SQ, NEWV = R + 3 * SQ, QNW = R + 4 * SQ, KNW = QNW + 1;
@@ -252,8 +258,8 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
         for (int db = 0; db < 8; ++db)
             va[db] = ring + kKeys * kRow + r * kRow + (((2 * db + ((c >> 1) & 1)) ^ (2 * r)) & 15) * 16 + 8 * (c & 1);
     }
-    const bool low = c >= R && c < 2 * R;       // a column of rounding remainders
-    const int cq = c < R ? c : low ? c - R : 0;  // the column's query row
+    const int part = c / R;                     // the column's part of the weights
+    const int cq = c < COLS ? c % R : 0;        // the column's query row
 #pragma unroll
     for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(va[i]));  // computed here, while the loads are in flight
 #pragma unroll
@@ -323,7 +329,7 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
         const U4 x = lds_read16(lds(&s.head[cq][(4 * kk + g) * 16])), zero = {0u, 0u, 0u, 0u};
-        qB[kk] = as_bf16x8(c < 2 * R ? x : zero);
+        qB[kk] = as_bf16x8(c < COLS ? x : zero);
     }
     // one past the column's last visible key: without a mask two tokens attend causally
     const int lim = SQ > 1 && !MASK ? L - SQ + cq / G + 1 : Lv;
@@ -381,15 +387,23 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
         for (int i = 0; i < 4; ++i) pw[i] = fexp2(x[i] - mx);
         l += (pw[0] + pw[1]) + (pw[2] + pw[3]);
         uint2 pp = {cvt_pk_bf16(pw[0], pw[1]), cvt_pk_bf16(pw[2], pw[3])};
-        const uint2 rest = {cvt_pk_bf16(pw[0] - bf16_lo(pp.x), pw[1] - bf16_hi(pp.x)),
-                            cvt_pk_bf16(pw[2] - bf16_lo(pp.y), pw[3] - bf16_hi(pp.y))};
-        pp.x = low ? rest.x : pp.x;
-        pp.y = low ? rest.y : pp.y;
+        bf16_rest(pw[0], pw[1], pp.x);
+        bf16_rest(pw[2], pw[3], pp.y);
+        const uint2 second = {cvt_pk_bf16(pw[0], pw[1]), cvt_pk_bf16(pw[2], pw[3])};
+        bf16_rest(pw[0], pw[1], second.x);
+        bf16_rest(pw[2], pw[3], second.y);
+        uint2 third = {cvt_pk_bf16(pw[0], pw[1]), cvt_pk_bf16(pw[2], pw[3])};
+        if constexpr (!THIRD) third = part == 0 ? third : uint2{0u, 0u};  // a product of its own
+        const uint2 rest = THIRD && part == 2 ? third : second;
+        pp = part == 0 ? pp : rest;
         const s16x4_t pv = __builtin_bit_cast(s16x4_t, pp);
 #pragma unroll
-        for (int db = 0; db < 8; ++db)
-            acc[db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4_t, lds_read_tr16(va[db] + slot)),
-                                                               pv, acc[db], 0, 0, 0);
+        for (int db = 0; db < 8; ++db) {
+            const s16x4_t v = __builtin_bit_cast(s16x4_t, lds_read_tr16(va[db] + slot));
+            acc[db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v, pv, acc[db], 0, 0, 0);
+            if constexpr (!THIRD)
+                acc[db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v, __builtin_bit_cast(s16x4_t, third), acc[db], 0, 0, 0);
+        }
     }
     // nothing of the wave's is in flight into LDS from here on (a mask can end the stream early)
     wait_loads<0>();
@@ -404,52 +418,43 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
             }
         }
     }
-    // the wave's state: the weight sums over its lane groups, the remainders' column added to
-    // its row's (unless the row holds an infinite sum, whose remainder may be 0 x inf), into the
-    // wave's own (drained) first stage; then the merge of the waves
+    // the wave's state: the weight sums over its lane groups and every column's accumulators, into
+    // the wave's own (drained) first stage; then the merge of the waves.  Dims 16 db + 4 g ... + 3
+    // of column c are chunk (4 db + g) ^ c of its 512 bytes: distinct banks for the columns.
     float lt = l + xor16(l);
     lt += xor32(lt);
-    float big = 0.f;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-#pragma unroll
-        for (int i = 0; i < 4; i += 2) big = fmaxf(fmaxf(__builtin_fabsf(acc[db][i]), __builtin_fabsf(acc[db][i + 1])), big);
-    const bool finite = __builtin_amdgcn_ballot_w64(c < R && big == INFINITY) == 0;
-    if (finite) {
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[db][i] += from_above<R>(acc[db][i]);
-    } else {
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float v = acc[db][i], r = from_above<R>(v);
-                acc[db][i] = __builtin_fabsf(v) < INFINITY ? v + r : v;
-            }
-    }
-    const uint32_t state = ring + c * 512 + g * 16;  // the column's floats: dims 16 db + 4 g ...
-    if (c < R) {
-        if (W > 1 && g == 0) {
-            s.ml[wave][c][0] = mx;
+    if (c < COLS) {
+        if (c < R && g == 0) {
+            if (W > 1) s.ml[wave][c][0] = mx;
             s.ml[wave][c][1] = lt;
         }
-        if (W == 1 && g == 0) s.ml[0][c][1] = lt;
+        const uint32_t state = ring + c * 512 + (g ^ c) * 16;
 #pragma unroll
         for (int db = 0; db < 8; ++db)
-            lds_write16(state + db * 64, __builtin_bit_cast(U4, acc[db]));
+            lds_write16(state ^ (db * 64), __builtin_bit_cast(U4, acc[db]));
     }
     lds_barrier();
     const int outputs = R * 32;  // of four dims
     for (int t = tid; t < outputs; t += W * 64) {
         const int r = t / 32, d = t % 32 * 4;
-        const uint32_t from = lds(&s.ring[0][0][0]) + r * 512 + d * 4;
+        const uint32_t from = lds(&s.ring[0][0][0]);
+        // a wave's four sums: the parts of the weights added up (unless a sum is infinite, whose
+        // remainder may be 0 x inf)
+        auto sums = [&](int w) {
+            auto column = [&](int c) {
+                return __builtin_bit_cast(f32x4_t, lds_read16(from + w * kStage + c * 512 + ((t % 32) ^ c) * 16));
+            };
+            f32x4_t a = column(r), rest = column(r + R);
+            if constexpr (THIRD) rest += column(r + 2 * R);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = __builtin_fabsf(a[i]) < INFINITY ? a[i] + rest[i] : a[i];
+            return a;
+        };
         float sl;
         f32x4_t sa;
         if constexpr (W == 1) {
             sl = s.ml[0][r][1];
-            sa = __builtin_bit_cast(f32x4_t, lds_read16(from));
+            sa = sums(0);
         } else {
             float mm = s.ml[0][r][0];
 #pragma unroll
@@ -460,7 +465,7 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
             for (int w = 0; w < W; ++w) {
                 const float wt = fexp2(s.ml[w][r][0] - mm);
                 sl += s.ml[w][r][1] * wt;
-                sa += __builtin_bit_cast(f32x4_t, lds_read16(from + w * kStage)) * wt;
+                sa += sums(w) * wt;
             }
         }
         const float inv = __builtin_amdgcn_rcpf(sl);

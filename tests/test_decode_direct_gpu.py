@@ -5,8 +5,9 @@ Against the float64 oracle (max-abs <= 2e-2, mean-abs <= 2e-3 for bf16 I/O with 
 accumulation) over one, four and eight waves per workgroup, with lengths on and around the
 16-key stages and the workgroup's whole stages, invalid positions, arenas read through
 offsets, and masks of every type that hide keys in the middle, at the end or all but one.
-The weights enter the products with 16 significant bits, so the result is as close to float64
-as the split kernel's float32 weights: its error norm is held to 1.02 times that kernel's."""
+The weights enter the products with all bits of their float32, so the result is as close to float64
+as the split kernel's: its error norm is held to 1.02 times that kernel's, and outputs whose terms
+cancel to what float32 weights leave."""
 import numpy as np
 import pytest
 import torch
@@ -19,7 +20,7 @@ from tests._util import assert_attention_close, bits, f64
 pytestmark = pytest.mark.gpu
 
 D = 128
-# (batch, kv_heads, capacity): one wave; one wave with two stages; four waves (256 pairs);
+# (batch, kv_heads, capacity): one wave; one wave with two stages; four waves (64 pairs and more);
 # eight waves, one stage to sixteen
 SHAPES = [(9, 8, 16), (5, 4, 32), (40, 8, 33), (64, 8, 300), (3, 8, 33), (7, 8, 130), (2, 2, 512), (5, 4, 1500), (2, 8, 2047)]
 
@@ -60,6 +61,27 @@ def test_attention_matches_the_oracle_and_the_split_kernel(pkg, device, batch, k
     assert_attention_close(f64(out)[ok], expected)
     error, reference = (np.linalg.norm(f64(x)[ok] - expected) for x in (out, split))
     assert error <= 1.02 * reference
+
+
+@pytest.mark.parametrize("group,tokens", [(1, 1), (2, 1), (4, 1), (2, 2), (4, 2)])
+@pytest.mark.parametrize("batch,kv_heads,capacity", [(64, 8, 16), (64, 8, 40), (7, 8, 40)])
+def test_cancelling_terms_keep_float32_weights(pkg, device, batch, kv_heads, capacity, group, tokens):
+    """|out - exact| <= 2^-8 |exact| (the output's rounding to bf16: half of 2^-7) + 2^-21 times the
+    mean |value| (float32 weights, sums and reciprocal: about 2^-23 each; the scores are kept small,
+    so their rounding adds less).  Weights of 16 bits are off by up to 2^-18 of it, which shows in
+    the outputs that cancel."""
+    gen = torch.Generator(device=device).manual_seed(capacity + group)
+    keys = torch.randn(batch, kv_heads, capacity, D, generator=gen, device=device, dtype=torch.bfloat16)
+    values = torch.randn(keys.shape, generator=gen, device=device, dtype=torch.bfloat16)
+    q = torch.randn(batch, tokens, kv_heads * group, D, generator=gen, device=device, dtype=torch.bfloat16) / 8
+    positions = tokens + torch.arange(batch) % 13
+    out = f64(pkg.decode_attention(q, keys, values, positions.to(device)))
+    for t in range(tokens):
+        last = positions.numpy() - tokens + 1 + t
+        exact = oatt.decode_attention(f64(q[:, t:t + 1]), f64(keys), f64(values), last, D ** -0.5)
+        size = oatt.decode_attention(f64(q[:, t:t + 1]), f64(keys), np.abs(f64(values)), last, D ** -0.5)
+        over = np.abs(out[:, t:t + 1] - exact) - (2.0 ** -8 * np.abs(exact) + 2.0 ** -21 * size)
+        assert over.max() <= 0, (over / size).max()
 
 
 @pytest.mark.parametrize("tokens", [1, 2])

@@ -338,8 +338,13 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
 #pragma unroll
     for (int db = 0; db < 8; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int t = 0; t < mine; ++t) {
-        // the next stage, into the slot scored last (the first two went out above)
-        if (issued < mine && issued <= t + 1) issue(issued++);
+        // the next stage, into the slot scored last (the first two went out above), once the wave's
+        // reads of that slot have returned: the products that use them order nothing against the
+        // loads, which the compiler does not see as writes of the slot
+        if (issued < mine && issued <= t + 1) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(issued++);
+        }
         if (issued > t + 1) wait_loads<kLoads>();
         else wait_loads<0>();
         const uint32_t slot = (t % kStages) * (W * kStage);

@@ -143,8 +143,9 @@ int q3t_rope_tables(const int64_t *positions, int64_t n, const float *inv_freq, 
  *     per request), one workgroup per (request, chunk, KV head); the default otherwise (the
  *     code predictor's 16-row caches, short arenas, few requests).  With max_chunks <= 0 and
  *     splits == 0, bf16 rows of 128 below 2048 keys, and unfused bf16 rows of 64 whose planes
- *     are short and few, run unsplit: one workgroup per (request, KV head); over
- *     bf16 rows of 128 it reads no key behind the last one that a mask shows.
+ *     are short and few, run unsplit: one workgroup per (request, KV head).  Over bf16 rows of
+ *     128 it stops at the last key that a request's mask shows: keys behind it are read only
+ *     within that key's 16 rows and the first 256, and none reaches the output, whatever it holds.
  * A request covered by several workgroups (balanced, chunked) merges their partial softmax
  * states through `workspace`; the last workgroup to finish writes the output.
  *

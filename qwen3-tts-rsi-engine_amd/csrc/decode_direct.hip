@@ -28,7 +28,9 @@
 // 64 requests x 16 rows 6.5 -> 3.8; 1 x 300 keys 10.7 -> 6.5; 21 x 30..511 keys 16.6 -> 9.4;
 // 64 x 32..511 keys 18.0 -> 15.4; 128 x 512 rows 32.0 -> 28.1; 1 x 1750 keys 22.5 -> 11.9.
 //   * masked launches bring the request's whole mask row into LDS once and stop at its last
-//     visible key: keys that the mask hides behind it are never read.
+//     visible key.  Each wave's first two stages are on their way before the mask is looked at, so
+//     of the keys that the mask hides behind it, those stages' are read and no others; none reaches
+//     the output, also where it is not finite: their scores are dropped and their value rows zeroed.
 #include "decode_params.hpp"
 
 namespace q3t {
@@ -356,6 +358,16 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
                 const uint32_t sb = ring + slot + r * kRow;
                 lds_write16(sb + ((c ^ r) & 15) * 16, lds_read16(lds(&s.head[NEWK + g][c * 16])));
                 lds_write16(sb + kKeys * kRow + ((c ^ (2 * r)) & 15) * 16, lds_read16(lds(&s.head[NEWV + g][c * 16])));
+            }
+        }
+        if constexpr (MASK) {
+            // value rows behind the last visible key: their weights are zero, but zero times an
+            // infinity or a NaN is not
+            if (w0 + kKeys > Lv) {
+                const U4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (w0 + 4 * i + g >= Lv) lds_write16(ring + slot + kKeys * kRow + (4 * i + g) * kRow + c * 16, zero);
             }
         }
         f32x4_t st = {0.f, 0.f, 0.f, 0.f};

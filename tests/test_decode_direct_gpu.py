@@ -143,7 +143,7 @@ def test_masks(pkg, device, batch, kv_heads, capacity, dtype, tokens):
     assert_attention_close(f64(out), expected)
 
 
-def test_a_masked_row_past_the_last_visible_key_is_not_read_and_infinite_values_stay(pkg, device):
+def test_infinite_values_of_visible_keys_stay(pkg, device):
     keys, values, q, _, _, _ = _problem(4, 8, 2, 200, 11, device)
     mask = (torch.arange(200, device=device) < 50).expand(4, 200)[:, None, None, :].contiguous()
     positions = torch.full((4,), 199, device=device, dtype=torch.int64)
@@ -155,6 +155,47 @@ def test_a_masked_row_past_the_last_visible_key_is_not_read_and_infinite_values_
     assert bool(torch.isposinf(out[..., 5]).all())
     keep = torch.arange(D, device=device) != 5
     assert torch.equal(out[..., keep], expected[..., keep])
+
+
+@pytest.mark.parametrize("tokens", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bool, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,kv_heads,capacity,visible", [
+    (5, 8, 30, [7, 16, 30, 1, 21]), (16, 8, 200, [50, 1, 64, 100, 199]), (5, 8, 300, [50, 129, 257, 3, 300]),
+    (2, 4, 1500, [70, 1003])])
+def test_keys_behind_the_last_visible_one_do_not_reach_the_output(pkg, device, batch, kv_heads, capacity, visible, dtype, tokens):
+    """One, four and eight waves; infinite keys and NaN values from the first hidden row on, of which
+    a wave's first stages are read: bit for bit the outputs over finite rows there."""
+    keys, values, q, _, _, _ = _problem(batch, kv_heads, 2, capacity, 17, device, tokens)
+    ends = torch.tensor([visible[b % len(visible)] for b in range(batch)])
+    seen = torch.arange(capacity) < ends[:, None]
+    mask = seen if dtype == torch.bool else torch.zeros(seen.shape, dtype=dtype).masked_fill(~seen, torch.finfo(dtype).min)
+    mask = mask.to(device)[:, None, None].expand(batch, 1, tokens, capacity).contiguous()
+    positions = torch.full((batch,), capacity - 1, device=device, dtype=torch.int64)
+    expected = pkg.decode_attention(q, keys, values, positions, mask=mask)
+    hidden = (~seen).to(device)[:, None, :, None]
+    out = pkg.decode_attention(q, keys.masked_fill(hidden, float("inf")), values.masked_fill(hidden, float("nan")),
+                               positions, mask=mask)
+    assert bool(torch.isfinite(expected).all()) and torch.equal(out, expected)
+
+
+@pytest.mark.parametrize("tokens", [1, 2])
+@pytest.mark.parametrize("batch,kv_heads,capacity", [(3, 8, 30), (16, 8, 131), (3, 8, 515)])
+def test_a_row_that_hides_every_key_is_nan_and_alone(pkg, device, batch, kv_heads, capacity, tokens):
+    """No weight to divide by: NaN, as on the split kernel; every other row as without that one."""
+    keys, values, q, _, _, _ = _problem(batch, kv_heads, 2, capacity, 19, device, tokens)
+    seen = torch.rand(batch, tokens, capacity, generator=torch.Generator().manual_seed(3)) < 0.5
+    seen[..., capacity // 2] = True
+    positions = torch.full((batch,), capacity - 1, device=device, dtype=torch.int64)
+    full = pkg.decode_attention(q, keys, values, positions, mask=seen.to(device)[:, None])
+    seen[1, tokens - 1] = False
+    out = pkg.decode_attention(q, keys, values, positions, mask=seen.to(device)[:, None])
+    split = pkg.decode_attention(q, keys, values, positions, mask=seen.to(device)[:, None], max_chunks=1)
+    assert bool(torch.isnan(out[1, tokens - 1]).all()) and bool(torch.isnan(split[1, tokens - 1]).all())
+    others = torch.ones(batch, tokens, dtype=torch.bool)
+    others[1] = False
+    assert torch.equal(out[others], full[others])
+    if tokens == 2:
+        assert_attention_close(f64(out[1, :1]), f64(full[1, :1]))
 
 
 def test_step_in_a_graph_follows_rewritten_positions(pkg, device):

@@ -234,6 +234,13 @@ Q3T_DEVICE void load_tile(i32x4_t rs, const uint32_t (&o)[N], uint32_t at, uint3
         load_to_lds16(rs, o[0] + at, base);
 }
 
+// 16 bytes to an address of 8-byte alignment, as output rows may have (a store of four dwords needs
+// dword alignment only).
+Q3T_DEVICE void store16_at8(char *p, const U4 &v) {
+    typedef uint32_t u32x4_at8_t __attribute__((ext_vector_type(4), aligned(8)));
+    *reinterpret_cast<u32x4_at8_t *>(p) = u32x4_at8_t{v.x, v.y, v.z, v.w};
+}
+
 Q3T_DEVICE void lds_write8(uint32_t byte_addr, uint32_t lo, uint32_t hi) {
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)byte_addr = u32x2_t{lo, hi};
@@ -694,7 +701,7 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
         for (int i = 0; i < 32 / RPL; ++i) {
             const int r = i * RPL + lr, pos = wq0 + r % QPW;
             const U4 v = lds_read16(rows + r * ROW + ((lc ^ r) & (CPR - 1)) * 16);
-            if (pos < n) store16(p.out + ((int64_t)(t0 + pos) * p.o_st + (hq0 + r / QPW) * p.o_sh) * 2 + lc * 16, v);
+            if (pos < n) store16_at8(p.out + ((int64_t)(t0 + pos) * p.o_st + (hq0 + r / QPW) * p.o_sh) * 2 + lc * 16, v);
         }
     }
 }

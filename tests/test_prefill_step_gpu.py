@@ -55,3 +55,21 @@ def test_short_requests(pkg, device, lengths, capacity, group, head_dim):
     ([66] * 65, 80)])                                                   # more than 64 requests
 def test_longer_requests(pkg, device, lengths, capacity, group, head_dim):
     _step(pkg, device, lengths, 8, group, head_dim, capacity, 5)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("lengths", [[45], [200], [400 + 7 * i for i in range(14)]])
+def test_output_rows_of_eight_byte_alignment(pkg, device, lengths, head_dim):
+    """An output that starts 8 bytes off a 16-byte boundary: the same rows, nothing around them."""
+    gen = torch.Generator(device=device).manual_seed(7)
+    total = sum(lengths)
+    q, k, v = (torch.randn(total, h, head_dim, generator=gen, device=device, dtype=torch.bfloat16) for h in (16, 8, 8))
+    cu = torch.tensor([0] + lengths).cumsum(0).to(device=device, dtype=torch.int32)
+    cos, sin = pkg.rope_tables(torch.cat([torch.arange(n) for n in lengths]).to(device), head_dim)
+    arena = torch.zeros(2, len(lengths), 8, max(lengths), head_dim, device=device, dtype=torch.bfloat16)
+    expected = pkg.prefill_step(q, k, v, cos, sin, cu, max(lengths), arena[0], arena[1])
+    flat = torch.full((expected.numel() + 8,), 7.0, device=device, dtype=torch.bfloat16)
+    out = flat[4:-4].view(expected.shape)
+    assert out.data_ptr() % 16 == 8
+    pkg.prefill_step(q, k, v, cos, sin, cu, max(lengths), arena[0], arena[1], out=out)
+    assert torch.equal(out, expected) and bool((flat[:4] == 7).all()) and bool((flat[-4:] == 7).all())

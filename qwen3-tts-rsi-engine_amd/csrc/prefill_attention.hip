@@ -328,7 +328,9 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
         qb = -1;
         b = 0;
         if (p.by_request) {
-            int before = blocks;  // blocks of requests 0 ... lane, then without the lane's own
+            // blocks of requests 0 ... lane; of a request longer than the caller said, those that the
+            // grid was sized for
+            int before = min(blocks, p.nqb);
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
                 const int y = __shfl_up(before, off);

@@ -73,3 +73,23 @@ def test_output_rows_of_eight_byte_alignment(pkg, device, lengths, head_dim):
     assert out.data_ptr() % 16 == 8
     pkg.prefill_step(q, k, v, cos, sin, cu, max(lengths), arena[0], arena[1], out=out)
     assert torch.equal(out, expected) and bool((flat[:4] == 7).all()) and bool((flat[-4:] == 7).all())
+
+
+@pytest.mark.parametrize("lengths,max_seqlen", [
+    ([150] + [126] * 60, 128),      # request by request
+    ([700] + [500] * 13, 512),      # by length
+    ([300, 90, 60], 96)])           # few workgroups
+def test_a_request_longer_than_max_seqlen_leaves_the_others_whole(pkg, device, lengths, max_seqlen):
+    """``max_seqlen`` bounds the lengths; rows past it are not attended.  Every other request's rows
+    are, as in a call that names the true maximum."""
+    gen = torch.Generator(device=device).manual_seed(11)
+    total = sum(lengths)
+    q, k, v = (torch.randn(total, h, 128, generator=gen, device=device, dtype=torch.bfloat16) for h in (16, 8, 8))
+    cu = torch.tensor([0] + lengths).cumsum(0).to(device=device, dtype=torch.int32)
+    cos, sin = pkg.rope_tables(torch.cat([torch.arange(n) for n in lengths]).to(device), 128)
+    arena = torch.zeros(2, len(lengths), 8, max(lengths), 128, device=device, dtype=torch.bfloat16)
+    expected = pkg.prefill_step(q, k, v, cos, sin, cu, max(lengths), arena[0], arena[1])
+    out = torch.zeros_like(expected)
+    pkg.prefill_step(q, k, v, cos, sin, cu, max_seqlen, arena[0], arena[1], out=out)
+    assert_attention_close(f64(out[:max_seqlen]), f64(expected[:max_seqlen]))
+    assert_attention_close(f64(out[lengths[0]:]), f64(expected[lengths[0]:]))

@@ -294,7 +294,7 @@ int q3t_decode_reset_workspace(void *workspace, int64_t workspace_bytes, void *s
  * (batch, 1, len_b, capacity) the causal rule is off: every key 0 ... capacity - 1 is scored
  * and the mask is added to the scaled scores, as SDPA adds an attention mask (the drop-in
  * path for any mask).  A query that sees no key gets a zero row.  max_seqlen bounds len_b;
- * query blocks past it are not computed.  bf16 only; head_dim 64 or 128;
+ * query blocks past it are not computed (their rows still reach the arena, new_values below).  bf16 only; head_dim 64 or 128;
  * q_heads / kv_heads in {1, 2, 4}.
  * Replaces: PrefillGraph.compute's padded causal attention (prefill_graph.py:31-50).
  */
@@ -328,8 +328,8 @@ typedef struct q3t_prefill_args {
     /* optional bf16 value rows (tokens, kv_heads, head_dim) of the step's tokens as the
        projection wrote them (strides in elements, 16-byte aligned): the products read key
        j's value of request b from token cu_seqlens[b] + j instead of `values`, and the
-       launch copies every token's row into `values` at its position (rows < capacity), the
-       value half of q3t_prefill_rope_write (which then runs with value == NULL).  Causal
+       launch copies every token's row into `values` at its position (rows < capacity; tokens past
+       cu_seqlens[batch] go on at the last request's next positions), the value half of q3t_prefill_rope_write (which then runs with value == NULL).  Causal
        launches only (mask == NULL): Q3T_EINVAL with a mask. */
     const void *new_values;
     int64_t nv_stride_t, nv_stride_h;

@@ -246,6 +246,32 @@ Q3T_DEVICE void lds_write8(uint32_t byte_addr, uint32_t lo, uint32_t hi) {
     *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)byte_addr = u32x2_t{lo, hi};
 }
 
+// Arena rows of one KV head for packed tokens that no query block covers: tokens t0 + pos0 ... t1 - 1
+// of a request starting at t0 keep their place, as the prologue gives them theirs.  Values, and
+// with RK the rotated keys.  A thread takes chunks ch and ch + CPR/2 of a row.
+template <int D, bool RK>
+Q3T_DEVICE void copy_uncovered_rows(const PrefillParams &p, int h, int64_t slot, int t0, int pos0, int64_t t1) {
+    constexpr int HALF = D / 16;  // chunks of half a row
+    const int64_t end = min(t1 - t0, p.cap);
+    for (int64_t pos = (int64_t)pos0 + threadIdx.x / HALF; pos < end; pos += 256 / HALF) {
+        const int ch = threadIdx.x % HALF;
+        const int64_t t = t0 + pos;
+        const char *v = p.nv + (t * p.nv_st + h * p.nv_sh) * 2 + ch * 16;
+        char *av = p.v + (slot * p.v_sb + h * p.v_sh + pos * p.v_st) * 2 + ch * 16;
+        store16(av, load16(v));
+        store16(av + D, load16(v + D));
+        if constexpr (RK) {
+            const char *k = p.nk + (t * p.nk_st + h * p.nk_sh) * 2 + ch * 16;
+            const char *cr = p.cs + t * p.cs_st * 2 + ch * 16, *sr = p.sn + t * p.cs_st * 2 + ch * 16;
+            char *ak = const_cast<char *>(p.k) + (slot * p.k_sb + h * p.k_sh + pos * p.k_st) * 2 + ch * 16;
+            U4 x1 = load16(k), x2 = load16(k + D), c1 = load16(cr), c2 = load16(cr + D), s1 = load16(sr), s2 = load16(sr + D), y1, y2;
+            rope8(&x1.x, &x2.x, &c1.x, &c2.x, &s1.x, &s2.x, &y1.x, &y2.x);
+            store16(ak, y1);
+            store16(ak + D, y2);
+        }
+    }
+}
+
 // MB: bytes per mask element (0: no mask, 2: bf16 / fp16, 4: fp32).  Without a mask the
 // causal rule (and the optional per-request key counts) bounds the key tiles of each query
 // block; with a mask every key tile of the view is scored and the mask alone decides, its
@@ -318,6 +344,16 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
     // (mbcnt), all wave-uniform, with no memory access beyond the row offsets.
     int b, qb, t0, n, kn;
     int64_t slot;
+    // one workgroup per KV head and query block writes the new rows into the arena
+    const bool writes = MB == 0 && p.nv && hq0 % p.group == 0;
+    if (writes && rest == 0) {
+        // tokens past the last request's end go on at its next positions
+        const int last = nb - 1;
+        const int from = nb <= 64 ? __builtin_amdgcn_readlane(start, last) : cu[last];
+        const int past = nb <= 64 ? __builtin_amdgcn_readlane(next, last) : cu[nb];
+        if (__builtin_expect(past < p.T && past >= from && from >= 0, false))
+            copy_uncovered_rows<D, RK>(p, h, slots ? slots[last] : last, from, past - from, p.T);
+    }
     if (nb <= 64) {
         int rows = 0, klen = 0;
         if (lane < nb) {
@@ -374,6 +410,8 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
     }
     const int q0 = qb * QB;
     if (q0 >= n) return;
+    // rows of a request longer than max_seqlen
+    if (__builtin_expect(writes && qb == p.nqb - 1 && n > q0 + QB, false)) copy_uncovered_rows<D, RK>(p, h, slot, t0, q0 + QB, (int64_t)t0 + n);
     // keys 0 ... kv_end-1 are visible to this block; the arena holds at most `cap` of them.
     // Causal: up to the block's last query and the request's key count; masked: every key.
     const int kv_end = MB ? (int)p.cap : (int)min((int64_t)min(min(n, kn), q0 + QB), p.cap);
@@ -476,8 +514,7 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
         rkc[u][2] = load16(p.sn + at);
         rkc[u][3] = load16(p.sn + at + D);
     };
-    // one workgroup per KV head and query block copies the values
-    const bool copy_values = own_values && !RK && hq0 % p.group == 0;
+    const bool copy_values = writes && !RK;
     if (copy_values) {
 #pragma unroll
         for (int i = 0; i < QPW / RPL; ++i)
@@ -651,7 +688,7 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
             rope8(&x1.x, &x2.x, &rkc[u][0].x, &rkc[u][1].x, &rkc[u][2].x, &rkc[u][3].x, &y1.x, &y2.x);
             lds_write16(k1, y1);
             lds_write16(k2, y2);
-            if (key >= q0 && hq0 % p.group == 0) {
+            if (key >= q0 && writes) {
                 char *ak = const_cast<char *>(p.k) + (slot * p.k_sb + h * p.k_sh + (int64_t)key * p.k_st) * 2 + rk_chunk * 16;
                 char *av = p.v + (slot * p.v_sb + h * p.v_sh + (int64_t)key * p.v_st) * 2 + rk_chunk * 16;
                 store16(ak, y1);

@@ -108,7 +108,9 @@ def prefill_step(query, key, value, cos, sin, cu_seqlens, max_seqlen, key_arena,
     Returns the attention output (T, Hq, D).  Two launches: the rotated keys into the arena,
     then attention, which rotates the queries as it loads them, reads the values from
     ``value`` and copies them into the arena.  One launch for short prompts (``max_seqlen`` up to
-    64), whose attention rotates the keys as well (q3t_prefill_step)."""
+    64), whose attention rotates the keys as well (q3t_prefill_step).  ``max_seqlen`` bounds the
+    requests' lengths: rows past it are not attended, but every token's key and value reach the
+    arena (those past ``cu_seqlens[-1]`` at the last request's next positions)."""
     write, _, device = _rope_write_args(query, key, None, cos, sin, cu_seqlens, key_arena, value_arena, kv_slots,
                                         None, False)
     attend, out, _, _ = prefill_args(query, key_arena, value_arena, cu_seqlens, max_seqlen, scale, kv_slots, out,

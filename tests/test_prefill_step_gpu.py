@@ -93,3 +93,25 @@ def test_a_request_longer_than_max_seqlen_leaves_the_others_whole(pkg, device, l
     pkg.prefill_step(q, k, v, cos, sin, cu, max_seqlen, arena[0], arena[1], out=out)
     assert_attention_close(f64(out[:max_seqlen]), f64(expected[:max_seqlen]))
     assert_attention_close(f64(out[lengths[0]:]), f64(expected[lengths[0]:]))
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("group", [1, 2, 4])
+@pytest.mark.parametrize("lengths,max_seqlen,past,capacity", [
+    ([20, 30], 32, 7, 64), ([200, 40, 0], 40, 3, 160), ([0], 8, 5, 16), ([30] * 70, 16, 90, 128),  # one launch
+    ([300, 100, 130], 128, 70, 260), ([150] + [126] * 60, 128, 1, 512), ([300] * 70, 100, 9, 320)])
+def test_every_token_reaches_the_arena(pkg, device, lengths, max_seqlen, past, capacity, group, head_dim):
+    """Tokens of requests longer than ``max_seqlen`` and past the last request's end: the arena bit for
+    bit the prologue's."""
+    gen = torch.Generator(device=device).manual_seed(13)
+    total, batch = sum(lengths) + past, len(lengths)
+    q, k, v = (torch.randn(total, 4 * h, head_dim, generator=gen, device=device, dtype=torch.bfloat16) for h in (group, 1, 1))
+    cu = torch.tensor([0] + lengths).cumsum(0).to(device=device, dtype=torch.int32)
+    cos, sin = pkg.rope_tables(torch.arange(total, device=device), head_dim)
+    slots = torch.randperm(batch, generator=torch.Generator().manual_seed(5)).to(device)
+    arena = torch.randn(2, batch, 4, capacity, head_dim, generator=gen, device=device, dtype=torch.bfloat16)
+    expected = arena.clone()
+    pkg.prefill_rope_write(q, k, v, cos, sin, cu, expected[0], expected[1], kv_slots=slots, rotate_query=False)
+    pkg.prefill_step(q, k, v, cos, sin, cu, max_seqlen, arena[0], arena[1], kv_slots=slots)
+    torch.cuda.synchronize()
+    assert torch.equal(arena.view(torch.int16), expected.view(torch.int16))

@@ -279,12 +279,16 @@ Q3T_DEVICE void copy_uncovered_rows(const PrefillParams &p, int h, int64_t slot,
 // values.  RK: the keys arrive unrotated (the step's own projection rows).  `cu`, `slots` and `nb`
 // lead the arguments: they are preloaded into scalar registers, so a wave asks for its row
 // offsets without waiting for the argument block.
-// SUB: 32-key blocks per tile.  One (three stages of 16 KiB, 168 VGPRs, three workgroups per CU)
-// where the launch fills the card; two (two stages of 32 KiB, the blocks' score chains independent
-// of one another, one maximum, barrier and wait for both) where it does not and the longest
-// block's chain of tiles is the launch: kFewGroups.
+// SUB: 32-key blocks per tile.  One (three stages of 16 KiB and the mask tile; without a mask 168
+// VGPRs and three workgroups per CU for two heads, else at most 256 and two) where the launch fills
+// the card; two (two stages of 32 KiB, the blocks' score chains independent of one another, one
+// maximum, barrier and wait for both) where it does not and the longest block's chain of tiles is
+// the launch: kFewGroups.  Three waves per SIMD asked of a masked instance, whose LDS does not let
+// them in, had the compiler keep to no bound: 276-280 registers, one workgroup per CU (us per layer,
+// so / with two asked for: 32 x 256 61.6 / 41.0, 16 x 512 98 / 59); one head without a mask spills
+// under it (32 prompts of 500 128 / 150).
 template <int D, int GH, int MB, int SUB, bool RK>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SUB == 2 || GH == 1 ? 2 : 3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SUB == 2 || GH == 1 || MB > 0 ? 2 : 3)))
 prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, PrefillParams p) {
     constexpr int QPW = 32 / GH;                  // queries per wave
     constexpr int QB = query_block(GH);           // queries per workgroup
@@ -807,18 +811,21 @@ extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void
 
 
 // Workgroups from which a launch fills the card (two per CU).  Below, the longest block's chain of
-// tiles bounds it.  us per layer, one / two 32-key blocks per tile: one prompt of 464 18.2 / 14.9 (64
-// workgroups), of 2048 58.2 / 41.0 (256), 8 x 256 under a mask 19.6 / 17.2; 16 prompts of 32..512
-// (664) 25.8 / 31.3, 8 of 1024..2048 92.9 / 97.1.
+// tiles bounds it.  us per layer, one / two 32-key blocks per tile: one prompt of 464 21.9 / 18.8 (64
+// workgroups), of 2048 58.2 / 41.0 (256); 16 prompts of 32..512 (664) 33.5 / 39.3, 8 of 1024..2048
+// 102.7 / 103.8.  Under a bf16 mask 8 x 256 16.1 / 14.8 (256), 2 x 1024 41.3 / 36.1 (256), 16 x 256
+// 25.3 / 25.2 (512), 32 x 256 41.0 / 40.7 (1024), 64 x 128 31.0 / 30.9; rows of 64 8 x 256 12.5 / 11.4
+// (256), 32 x 256 25.7 / 28.2 (1024).
+// Two blocks' mask rows cost their gain where they leave one workgroup on a CU: fp32 masks (8 x 256
+// 15.7 / 16.9, 16 x 256 25.9 / 36.1, 2 x 1024 38.4 / 42.8; rows of 64 8 x 256 11.6 / 12.5) and one head's
+// rows of 128 under a mask (8 x 256 16.7 / 17.2, 16 x 256 25.2 / 34.4) always take one.
 constexpr int64_t kFewGroups = 512;
 // Bytes of one KV head's rows of the whole step from which its L2 share no longer holds them.
 constexpr int64_t kL2Rows = 3 << 20;
 
-template <int D, int GH, int SUB>
-static void launch_mask(const PrefillParams &p, const int64_t *slots, dim3 grid, hipStream_t s) {
-    if (!p.mask) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 0, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
-    else if (p.mdt == Q3T_F32) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 4, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
-    else hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 2, SUB, false>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
+template <int D, int GH, int MB, int SUB, bool RK = false>
+static void launch_tiles(const PrefillParams &p, const int64_t *slots, dim3 grid, hipStream_t s) {
+    hipLaunchKernelGGL((prefill_attention_kernel<D, GH, MB, SUB, RK>), grid, dim3(256), 0, s, p.cu, slots, p.B, p);
 }
 
 template <int D, int GH>
@@ -844,9 +851,15 @@ static void launch_prefill(const PrefillParams &p, int64_t max_seqlen, const int
     // prompts of 500 85.9 / 79.2, 16 of 512 52.5 / 46.4, 8 of 1024..2048 93.7 / 103).
     q.by_request = p.T * D * 4 > kL2Rows && (int64_t)q.nqb * 8 <= (p.T + QB - 1) / QB;
     const dim3 grid((uint32_t)wgs);
-    if (p.nk) hipLaunchKernelGGL((prefill_attention_kernel<D, GH, 0, 2, true>), grid, dim3(256), 0, s, p.cu, slots, p.B, q);
-    else if (wgs <= kFewGroups) launch_mask<D, GH, 2>(q, slots, grid, s);
-    else launch_mask<D, GH, 1>(q, slots, grid, s);
+    const bool few = wgs <= kFewGroups;
+    if (p.nk) launch_tiles<D, GH, 0, 2, true>(q, slots, grid, s);
+    else if (p.mask && p.mdt == Q3T_F32) launch_tiles<D, GH, 4, 1>(q, slots, grid, s);
+    else if (p.mask) {
+        if constexpr (D == 128 && GH == 1) launch_tiles<D, GH, 2, 1>(q, slots, grid, s);
+        else if (few) launch_tiles<D, GH, 2, 2>(q, slots, grid, s);
+        else launch_tiles<D, GH, 2, 1>(q, slots, grid, s);
+    } else if (few) launch_tiles<D, GH, 0, 2>(q, slots, grid, s);
+    else launch_tiles<D, GH, 0, 1>(q, slots, grid, s);
 }
 
 static int launch_prefill_sizes(const PrefillParams &p, int64_t head_dim, int64_t max_seqlen, const int64_t *slots, hipStream_t s) {

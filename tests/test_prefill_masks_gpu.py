@@ -61,6 +61,31 @@ def test_masked_prefill_padded_batch(pkg, device, dtype):
     assert_attention_close(f64(out), expected)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(16, 8, 128), (16, 16, 128), (16, 4, 128), (16, 8, 64), (16, 16, 64)])
+@pytest.mark.parametrize("batch,length", [(17, 249), (9, 250), (70, 128), (3, 65)])
+def test_masked_prefill_below_and_above_a_full_card(pkg, device, batch, length, q_heads, kv_heads, head_dim, dtype):
+    """More than 512 workgroups (tiles of one 32-key block) and fewer (two blocks, where the mask's
+    type allows), more than 64 requests; causal rows, a random half and rows that hide every key
+    (zero rows) against float64."""
+    gen = torch.Generator(device=device).manual_seed(length)
+    keys = (length + 7) // 8 * 8
+    q = torch.randn(batch, length, q_heads, head_dim, generator=gen, device=device, dtype=torch.bfloat16)
+    k = torch.randn(batch, kv_heads, keys, head_dim, generator=gen, device=device, dtype=torch.bfloat16)
+    v = torch.randn(k.shape, generator=gen, device=device, dtype=torch.bfloat16)
+    seen = torch.ones(batch, length, keys, device=device, dtype=torch.bool).tril()
+    seen[1::2] = torch.rand(seen[1::2].shape, generator=gen, device=device) < 0.5
+    seen[0, length // 2], seen[-1, -1] = False, False
+    mask = torch.zeros(seen.shape, device=device, dtype=dtype).masked_fill(~seen, float("-inf"))[:, None]
+    cu = torch.arange(0, (batch + 1) * length, length, dtype=torch.int32, device=device)
+    out = pkg.prefill_attention(q.view(-1, q_heads, head_dim), k, v, cu, length, mask=mask).view(q.shape)
+    for b in range(batch):
+        kb, vb = (x[b].double().repeat_interleave(q_heads // kv_heads, 0) for x in (k, v))
+        scores = torch.bmm(q[b].double().transpose(0, 1).contiguous(), kb.transpose(1, 2).contiguous()) * head_dim ** -0.5
+        weights = torch.nan_to_num(scores.masked_fill(~seen[b], float("-inf")).softmax(-1))
+        assert_attention_close(f64(out[b]), torch.bmm(weights, vb).transpose(0, 1).cpu().numpy())
+
+
 def test_key_counts_equal_the_padded_mask(pkg, device):
     """kv_lens gives PrefillGraph's key-valid and causal rule without a mask tensor: the same
     result as the masked kernel and the oracle, padding rows included."""

@@ -5,7 +5,7 @@
 // prefill KV is later copied into the request's arena slot (continuous.py:468-471,
 // packed_kv.py:6-31).  Here requests are packed along the token axis by cu_seqlens, so
 // only valid rows exist, and rotated keys/values go straight into the arena slot.
-#include "q3t_common.hpp"
+#include "prefill_params.hpp"
 
 namespace q3t {
 
@@ -149,72 +149,9 @@ __global__ void __launch_bounds__(256) prefill_rope_write_kernel(PrefillRopeWrit
 // the keys.  The running maximum moves only when a step's maximum exceeds it by more than
 // kRescaleLog2 (log2 units), so the accumulators are rescaled rarely and unnormalised weights
 // stay below 2^kRescaleLog2 (well inside bf16 and fp32 range).
-constexpr int kXcds = 8;        // MI355X: 8 XCDs of 32 CUs
-constexpr int kCusPerXcd = 32;
-constexpr int kKeys = 32;     // keys of one MFMA block of scores
-constexpr float kLog2eP = 1.4426950408889634f;
-constexpr float kRescaleLog2 = 8.0f;
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // Queries per workgroup.
 constexpr int query_block(int gh) { return 4 * (32 / gh); }
-
-struct PrefillParams {
-    int B, Hq, Hkv, nqb, group;
-    int64_t T;
-    float scale_log2;
-    const int32_t *cu;
-    const char *q;
-    int64_t q_st, q_sh;
-    const char *k;
-    char *v;  // written only with nv
-    int64_t k_sb, k_sh, k_st, v_sb, v_sh, v_st;
-    int64_t cap;
-    const int64_t *slots;
-    char *out;
-    int64_t o_st, o_sh;
-    const char *cs, *sn;  // optional cos/sin rows per token: the query rows are rotated on load
-    int64_t cs_st;
-    const int32_t *kvl;   // optional keys per request (a right-padded batch): query i sees keys
-                          // j <= i with j < kvl[b]
-    const char *mask;     // optional (B, 1, Lq, capacity) additive mask: every key is scored
-    int mdt;              // mask element type (Q3T_BF16, Q3T_F16 or Q3T_F32)
-    int64_t m_sb, m_sq;   // mask strides (elements) of requests and query rows; keys unit-stride
-    // optional value rows of the step's tokens as the projection wrote them: the products
-    // read them (key j of request b is token cu[b] + j) and each workgroup copies those of its
-    // query block into the arena view `v` at their positions
-    const char *nv;
-    int64_t nv_st, nv_sh;
-    // key rows of the step's tokens before their rotation: the launch rotates each tile in LDS
-    // and writes its block's rows into the arena (instances that rotate keys only)
-    const char *nk;
-    int64_t nk_st, nk_sh;
-    int by_request;       // work items numbered request by request
-};
-
-constexpr float kEmptyP = -1.0e30f;  // finite running maximum before any visible key (masked)
-
-// 16 bytes of a mask tile row in LDS -> 4 (2-byte types) or 2 x 2 (fp32: two reads) values in
-// log2 units; positive infinity never occurs in an additive mask, -inf (and finfo.min, which
-// overflows to -inf once scaled) gives a zero weight.
-template <int MB>
-Q3T_DEVICE void mask_values(uint32_t addr, int mdt, float (&mv)[4]) {
-    if constexpr (MB == 2) {
-        typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-        const u32x2_t w = *(__attribute__((address_space(3))) const u32x2_t *)(uintptr_t)addr;
-        const uint32_t h[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float v = mdt == Q3T_F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)h[i])
-                                           : bf16_to_float(h[i]);
-            mv[i] = v * kLog2eP;
-        }
-    } else {
-        const U4 w = lds_read16(addr);
-        const uint32_t f[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mv[i] = __uint_as_float(f[i]) * kLog2eP;
-    }
-}
 
 // A wave's share of a tile's K or V rows: N loads of 1 KiB, consecutive in LDS.
 template <int N>
@@ -244,32 +181,6 @@ Q3T_DEVICE void store16_at8(char *p, const U4 &v) {
 Q3T_DEVICE void lds_write8(uint32_t byte_addr, uint32_t lo, uint32_t hi) {
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)byte_addr = u32x2_t{lo, hi};
-}
-
-// Arena rows of one KV head for packed tokens that no query block covers: tokens t0 + pos0 ... t1 - 1
-// of a request starting at t0 keep their place, as the prologue gives them theirs.  Values, and
-// with RK the rotated keys.  A thread takes chunks ch and ch + CPR/2 of a row.
-template <int D, bool RK>
-Q3T_DEVICE void copy_uncovered_rows(const PrefillParams &p, int h, int64_t slot, int t0, int pos0, int64_t t1) {
-    constexpr int HALF = D / 16;  // chunks of half a row
-    const int64_t end = min(t1 - t0, p.cap);
-    for (int64_t pos = (int64_t)pos0 + threadIdx.x / HALF; pos < end; pos += 256 / HALF) {
-        const int ch = threadIdx.x % HALF;
-        const int64_t t = t0 + pos;
-        const char *v = p.nv + (t * p.nv_st + h * p.nv_sh) * 2 + ch * 16;
-        char *av = p.v + (slot * p.v_sb + h * p.v_sh + pos * p.v_st) * 2 + ch * 16;
-        store16(av, load16(v));
-        store16(av + D, load16(v + D));
-        if constexpr (RK) {
-            const char *k = p.nk + (t * p.nk_st + h * p.nk_sh) * 2 + ch * 16;
-            const char *cr = p.cs + t * p.cs_st * 2 + ch * 16, *sr = p.sn + t * p.cs_st * 2 + ch * 16;
-            char *ak = const_cast<char *>(p.k) + (slot * p.k_sb + h * p.k_sh + pos * p.k_st) * 2 + ch * 16;
-            U4 x1 = load16(k), x2 = load16(k + D), c1 = load16(cr), c2 = load16(cr + D), s1 = load16(sr), s2 = load16(sr + D), y1, y2;
-            rope8(&x1.x, &x2.x, &c1.x, &c2.x, &s1.x, &s2.x, &y1.x, &y2.x);
-            store16(ak, y1);
-            store16(ak + D, y2);
-        }
-    }
 }
 
 // MB: bytes per mask element (0: no mask, 2: bf16 / fp16, 4: fp32).  Without a mask the
@@ -323,97 +234,17 @@ prefill_attention_kernel(const int32_t *cu, const int64_t *slots, int nb, Prefil
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hi = lane >> 5, col = lane & 31;
     const int hgroups = p.Hq / GH;
-    // Placement: the hardware deals workgroup i to XCD i % 8 and, within an XCD, to its 32 CUs
-    // in turn, so CU k of an XCD holds the XCD's workgroups k, k + 32, k + 64 at once (three
-    // per CU).  Work items are numbered longest first; reversing the order within the second
-    // and third of every four rounds of 32 puts a short item next to every long one on a CU.
-    // Measured on the 16-prompt workload (seed 0): the most loaded CU from 27 to 20 tiles.
-    const int wg = [&] {
-        const int xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
-        const int rounds = (int)gridDim.x / (kXcds * kCusPerXcd);  // complete rounds on every XCD
-        if (j >= rounds * kCusPerXcd) return (int)blockIdx.x;
-        const int r = j / kCusPerXcd, pos = j % kCusPerXcd;
-        const bool flip = (r & 3) == 1 || (r & 3) == 2;
-        return (r * kCusPerXcd + (flip ? kCusPerXcd - 1 - pos : pos)) * kXcds + xcd;
-    }();
+    const int wg = place_workgroup(blockIdx.x, gridDim.x);
     const int hq0 = (wg % hgroups) * GH;  // the workgroup's first query head
     const int h = hq0 / p.group;          // the workgroup's KV head
     const int rest = wg / hgroups;
-    // Work item `rest` of this head group: a (query block qb, request b) pair, numbered with
-    // the longest blocks first.  Up to 64 requests the numbering is dense: only pairs with
-    // rows exist, so the grid's round-robin placement over shader engines sees real work
-    // evenly (empty slots in between would pile long blocks onto some engines and stall the
-    // in-order dispatch behind them).  Lane i holds request i's row range; each level counts
-    // the requests with a block there (ballot) and the item's request is picked by rank
-    // (mbcnt), all wave-uniform, with no memory access beyond the row offsets.
-    int b, qb, t0, n, kn;
-    int64_t slot;
     // one workgroup per KV head and query block writes the new rows into the arena
     const bool writes = MB == 0 && p.nv && hq0 % p.group == 0;
-    if (writes && rest == 0) {
-        // tokens past the last request's end go on at its next positions
-        const int last = nb - 1;
-        const int from = nb <= 64 ? __builtin_amdgcn_readlane(start, last) : cu[last];
-        const int past = nb <= 64 ? __builtin_amdgcn_readlane(next, last) : cu[nb];
-        if (__builtin_expect(past < p.T && past >= from && from >= 0, false))
-            copy_uncovered_rows<D, RK>(p, h, slots ? slots[last] : last, from, past - from, p.T);
-    }
-    if (nb <= 64) {
-        int rows = 0, klen = 0;
-        if (lane < nb) {
-            rows = (start < 0 || start >= p.T) ? 0 : (int)min((int64_t)(next - start), p.T - start);
-            klen = p.kvl ? p.kvl[lane] : rows;
-        }
-        const int blocks = rows > 0 ? (rows + QB - 1) / QB : 0;
-        qb = -1;
-        b = 0;
-        if (p.by_request) {
-            // blocks of requests 0 ... lane; of a request longer than the caller said, those that the
-            // grid was sized for
-            int before = min(blocks, p.nqb);
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int y = __shfl_up(before, off);
-                if (lane >= off) before += y;
-            }
-            const uint64_t done = __builtin_amdgcn_ballot_w64(before <= rest);  // requests wholly before the item
-            if (~done) {
-                b = __builtin_ctzll(~done);
-                qb = __builtin_amdgcn_readlane(before, b) - 1 - rest;
-            }
-        } else {
-            int remaining = rest;
-            for (int level = p.nqb - 1; level >= 0; --level) {
-                const uint64_t has = __builtin_amdgcn_ballot_w64(blocks > level);
-                const int count = __builtin_popcountll(has);
-                if (remaining < count) {
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0u));
-                    const uint64_t pick = __builtin_amdgcn_ballot_w64(blocks > level && (int)rank == remaining);
-                    b = __builtin_ctzll(pick);
-                    qb = level;
-                    break;
-                }
-                remaining -= count;
-            }
-        }
-        if (qb < 0) return;  // past the last block with rows
-        t0 = __builtin_amdgcn_readlane(start, b);
-        n = __builtin_amdgcn_readlane(rows, b);
-        kn = __builtin_amdgcn_readlane(klen, b);
-        slot = ((int64_t)__builtin_amdgcn_readlane((int)(slot_l >> 32), b) << 32) |
-               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)slot_l, b);
-    } else {
-        b = rest % p.B;
-        qb = p.nqb - 1 - rest / p.B;  // the longest blocks are dispatched first
-        t0 = cu[b];
-        if (t0 < 0 || t0 >= p.T) return;
-        n = (int)min((int64_t)(cu[b + 1] - t0), p.T - t0);  // rows past the packed tokens do not exist
-        kn = p.kvl ? p.kvl[b] : n;
-        slot = slots ? slots[b] : b;
-    }
-    const int q0 = qb * QB;
-    if (q0 >= n) return;
+    if (writes && rest == 0) copy_rows_past_the_end<D, RK>(p, cu, slots, nb, start, next, h);
+    PrefillItem item;
+    if (!find_item<QB>(p, cu, slots, nb, start, next, slot_l, rest, item)) return;
+    const int b = item.b, qb = item.qb, t0 = item.t0, n = item.n, kn = item.kn, q0 = qb * QB;
+    const int64_t slot = item.slot;
     // rows of a request longer than max_seqlen
     if (__builtin_expect(writes && qb == p.nqb - 1 && n > q0 + QB, false)) copy_uncovered_rows<D, RK>(p, h, slot, t0, q0 + QB, (int64_t)t0 + n);
     // keys 0 ... kv_end-1 are visible to this block; the arena holds at most `cap` of them.
@@ -820,6 +651,18 @@ extern "C" int q3t_prefill_rope_write(const q3t_prefill_rope_write_args *a, void
 // 15.7 / 16.9, 16 x 256 25.9 / 36.1, 2 x 1024 38.4 / 42.8; rows of 64 8 x 256 11.6 / 12.5) and one head's
 // rows of 128 under a mask (8 x 256 16.7 / 17.2, 16 x 256 25.2 / 34.4) always take one.
 constexpr int64_t kFewGroups = 512;
+// One-head groups take blocks of 64 queries on 16-column products (prefill_narrow.hip) where the query
+// rows of all heads are fewer than this many blocks of 128 would hold; there the chain of the longest
+// block is the launch, and a wave's is half as long.  us per layer, blocks of 128 / of 64 (16 heads
+// unless said): one prompt of 464 20.7 / 19.8, 8 x 250 23.9 / 22.9 (250 blocks), 8 heads 16 of 32..512
+// 28.5 / 27.4 (300), 12 x 500 32.8 / 32.1 (375), 16 x 500 39.5 / 42.2 (500), rows of 64 12 x 500 21.9 /
+// 20.7 and 16 x 500 25.4 / 26.0; bf16 mask 2 x 1024 42.1 / 40.0 (256), 12 x 256 22.3 / 26.9 (384), rows of
+// 64 14.1 / 13.4, 8 x 512 23.7 / 25.4 (512); fp32 mask, one workgroup of 128 per CU, 12 x 256 30.9 / 26.4,
+// 8 x 512 51.3 / 45.2 (512), 16 x 256 34.0 / 34.8, 32 x 256 62.1 / 66.0 (1024).
+static bool narrow_blocks(const PrefillParams &p, int head_dim, int64_t wgs) {
+    const int64_t blocks = !p.mask || head_dim == 64 ? 384 : p.mdt == Q3T_F32 ? 512 : 256;
+    return p.T * p.Hq <= blocks * 128 && wgs <= 16 * blocks;  // the grid too: requests of no rows count in it
+}
 // Bytes of one KV head's rows of the whole step from which its L2 share no longer holds them.
 constexpr int64_t kL2Rows = 3 << 20;
 
@@ -833,16 +676,12 @@ static void launch_prefill(const PrefillParams &p, int64_t max_seqlen, const int
     constexpr int QB = query_block(GH);
     PrefillParams q = p;
     q.nqb = (int)((max_seqlen + QB - 1) / QB);
-    const int64_t hgroups = p.Hq / GH;
-    int64_t wgs = (int64_t)p.B * q.nqb * hgroups;
-    // items are numbered densely up to 64 requests: a request of L rows has ceil(L / QB) blocks,
-    // so there are at most (T + (QB - 1) B) / QB of them; rounded up to whole rounds of one
-    // workgroup per CU, which keeps the placement of every item as in the full grid
-    const int64_t items = (p.T + (int64_t)(QB - 1) * p.B) / QB;
-    if (p.B <= 64) {
-        const int64_t round = kXcds * kCusPerXcd;
-        const int64_t bound = (items * hgroups + round - 1) / round * round;
-        if (bound < wgs) wgs = bound;
+    const int64_t wgs = prefill_workgroups(p, QB, p.Hq / GH, max_seqlen);
+    if constexpr (GH == 1) {
+        if (!p.nk && narrow_blocks(p, D, wgs)) {
+            launch_prefill_narrow(p, D, max_seqlen, s);
+            return;
+        }
     }
     // Longest blocks first over all requests ends the launch evenly, but every request's rows are
     // then in use at once; request by request keeps the rows in use in the XCD's L2.  The latter

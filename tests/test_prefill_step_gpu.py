@@ -58,6 +58,14 @@ def test_longer_requests(pkg, device, lengths, capacity, group, head_dim):
 
 
 @pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("kv_heads,lengths,capacity", [
+    (2, [66] * 65, 80), (2, [65, 300, 0, 129, 512, 64], 300), (1, [2000], 2048),    # blocks of 64 queries
+    (8, [512] * 9, 512)])                                                            # of 128
+def test_one_head_groups(pkg, device, kv_heads, lengths, capacity, head_dim):
+    _step(pkg, device, lengths, kv_heads, 1, head_dim, capacity, 9)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("lengths", [[45], [200], [400 + 7 * i for i in range(14)]])
 def test_output_rows_of_eight_byte_alignment(pkg, device, lengths, head_dim):
     """An output that starts 8 bytes off a 16-byte boundary: the same rows, nothing around them."""

@@ -157,10 +157,10 @@ decode_chunks_kernel(DecodeParams p) {
     const int rest = blockIdx.x / p.Hkv;
     const int c = rest % p.nchunks, b = rest / p.nchunks;
 
-    const int64_t pb = p.pos ? p.pos[b] : p.ctx - 1;
+    const int64_t pb = p.pos[b];
     Work work;
     work.load_rows(p, b, h);
-    const int L = (pb >= 0 && pb < p.ctx) ? (int)pb + 1 : 0;
+    const int L = keys_of(p, pb);
     if (L == 0) {  // no valid position: attends nothing, zero rows (written by chunk 0)
         if (c == 0) Work::write_zeros(p, b, h);
         return;
@@ -230,8 +230,8 @@ decode_balanced_kernel(DecodeParams p) {
             const int b = tid * per + e;
             w[e] = 0;
             if (e < per && b < p.B) {
-                const int64_t pb = p.pos ? p.pos[b] : p.ctx - 1;
-                const int L = (pb >= 0 && pb < p.ctx) ? (int)pb + 1 : 0;
+                const int64_t pb = p.pos[b];
+                const int L = keys_of(p, pb);
                 sm_len[b] = L;
                 w[e] = L > 0 ? L : 1;
             }
@@ -477,11 +477,11 @@ __global__ void __launch_bounds__(kThreads) decode_bundled_kernel(const int32_t 
         int64_t pb[2] = {-1, -1};
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-            if (lane + 64 * e < p.B) pb[e] = p.pos ? p.pos[lane + 64 * e] : p.ctx - 1;
+            if (lane + 64 * e < p.B) pb[e] = p.pos[lane + 64 * e];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int b = lane + 64 * e;
-            const int L = (pb[e] >= 0 && pb[e] < p.ctx) ? (int)pb[e] + 1 : 0;
+            const int L = keys_of(p, pb[e]);
             len[e] = L;
             key[e] = b < p.B ? (L << 10) | (1023 - b) : -1;
             s.keys[wave][b] = key[e];
@@ -1115,10 +1115,10 @@ static int dispatch_sq(const DecodeParams &p, int sq, bool fused, hipStream_t s)
     if (fused) {
         if constexpr (sizeof(T) == 2 && D == 128) {
             if (sq == 1) {
-                if (p.has_mask) launch_decode<T, D, G, 1, true, true>(p, s);
+                if (p.mask) launch_decode<T, D, G, 1, true, true>(p, s);
                 else launch_decode<T, D, G, 1, true, false>(p, s);
             } else if (sq == 2) {
-                if (p.has_mask) launch_decode<T, D, G, 2, true, true>(p, s);
+                if (p.mask) launch_decode<T, D, G, 2, true, true>(p, s);
                 else launch_decode<T, D, G, 2, true, false>(p, s);
             } else {
                 return Q3T_EUNSUPPORTED;
@@ -1129,10 +1129,10 @@ static int dispatch_sq(const DecodeParams &p, int sq, bool fused, hipStream_t s)
         }
     }
     if (sq == 1) {
-        if (p.has_mask) launch_decode<T, D, G, 1, false, true>(p, s);
+        if (p.mask) launch_decode<T, D, G, 1, false, true>(p, s);
         else launch_decode<T, D, G, 1, false, false>(p, s);
     } else if (sq == 2) {
-        if (p.has_mask) launch_decode<T, D, G, 2, false, true>(p, s);
+        if (p.mask) launch_decode<T, D, G, 2, false, true>(p, s);
         else launch_decode<T, D, G, 2, false, false>(p, s);
     } else {
         return Q3T_EUNSUPPORTED;
@@ -1148,6 +1148,21 @@ static int dispatch_g(const DecodeParams &p, int g, int sq, bool fused, hipStrea
         case 4: return dispatch_sq<T, D, 4>(p, sq, fused, s);
         default: return Q3T_EUNSUPPORTED;
     }
+}
+
+// Memory that the positions of a call without any are loaded from (their values are not used), per
+// device; its address is looked up once.
+static __device__ int64_t no_positions[kMaxBatch];
+constexpr int kMaxDevices = 64;
+static const int64_t *any_positions() {
+    static std::mutex mutex;
+    static const int64_t *found[kMaxDevices];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lock(mutex);
+    void *ptr = nullptr;
+    if (!found[dev] && hipGetSymbolAddress(&ptr, HIP_SYMBOL(no_positions)) == hipSuccess) found[dev] = (const int64_t *)ptr;
+    return found[dev];
 }
 
 // Host-side validation and parameter set-up shared by every decode entry point; the device
@@ -1197,7 +1212,6 @@ static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, Deco
     p.bundles = grid == Q3T_GRID_BUNDLED ? (int)bundle_count(a) : 0;
     p.stream = stream_kv(a->batch, a->kv_heads, a->ctx, a->head_dim * es);
     p.scale_log2 = a->scale * kLog2e;
-    p.has_mask = a->mask != nullptr;
     p.mask_dtype = (int)a->mask_dtype;
     p.q = (const char *)a->query;
     p.q_sb = a->q_stride_b; p.q_ss = a->q_stride_s; p.q_sh = a->q_stride_h;
@@ -1205,7 +1219,9 @@ static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, Deco
     p.k_sb = a->k_stride_b; p.k_sh = a->k_stride_h; p.k_st = a->k_stride_t;
     p.v_sb = a->v_stride_b; p.v_sh = a->v_stride_h; p.v_st = a->v_stride_t;
     p.offs = a->kv_offsets;
-    p.pos = all_keys ? nullptr : a->positions;
+    p.pos = a->positions;
+    if (all_keys && !(p.pos = any_positions())) return (int)hipErrorInvalidDevicePointer;
+    p.pos_limit = all_keys ? 0 : (int)a->ctx;
     p.mask = (const char *)a->mask;
     p.m_sb = a->mask_stride_b; p.m_ss = a->mask_stride_s; p.m_st = a->mask_stride_t;
     p.out = (char *)a->out;
@@ -1280,7 +1296,6 @@ extern "C" int q3t_decode_reset_workspace(void *workspace, int64_t workspace_byt
 constexpr int64_t kScratchBytes = 8 << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 
-constexpr int kMaxDevices = 64;
 static std::mutex scratch_mutex;
 static char *scratch_ptr[kMaxDevices];
 

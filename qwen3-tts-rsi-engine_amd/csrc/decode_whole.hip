@@ -25,10 +25,10 @@ __global__ void __launch_bounds__(kWholeWaves * 64) decode_whole_kernel(DecodePa
     __shared__ typename Work::Lds lds;
     __shared__ typename Work::NewRows snew;
     const int h = blockIdx.x % p.Hkv, b = blockIdx.x / p.Hkv;
-    const int64_t pb = p.pos ? p.pos[b] : p.ctx - 1;
+    const int64_t pb = p.pos[b];
     Work work;
     work.load_rows(p, b, h);
-    const int L = (pb >= 0 && pb < p.ctx) ? (int)pb + 1 : 0;
+    const int L = keys_of(p, pb);
     if (L == 0) {
         Work::write_zeros(p, b, h);
         return;
@@ -50,10 +50,10 @@ static void launch_one(const DecodeParams &p, hipStream_t s) {
 template <typename T, int D, int G>
 static void launch(const DecodeParams &p, int tokens, hipStream_t s) {
     if (tokens == 1) {
-        if (p.has_mask) launch_one<T, D, G, 1, true>(p, s);
+        if (p.mask) launch_one<T, D, G, 1, true>(p, s);
         else launch_one<T, D, G, 1, false>(p, s);
     } else if constexpr (G <= 2) {  // eight query rows do not fit a wave's registers
-        if (p.has_mask) launch_one<T, D, G, 2, true>(p, s);
+        if (p.mask) launch_one<T, D, G, 2, true>(p, s);
         else launch_one<T, D, G, 2, false>(p, s);
     }
 }

@@ -83,7 +83,8 @@ int q3t_copy_strided(void *dst, const void *src, int64_t elem_size, int ndim,
 /*
  * A larger copy of a contiguous arena of planes * slots * heads blocks: each block of dst
  * (new_bytes) gets the old block's old_bytes and zeros after them; blocks of slots `used` and
- * past it get zeros.  Q3T_EUNSUPPORTED unless blocks and pointers are 16-byte multiples.
+ * past it get zeros.  Q3T_EUNSUPPORTED unless blocks and pointers are 16-byte multiples
+ * and the blocks, 16 KiB a workgroup, take fewer than 2^24 workgroups.
  * Replaces: ensure_capacity's allocation and copy (continuous.py:353-363).
  */
 int q3t_grow_arena(void *dst, const void *src, int64_t planes, int64_t slots, int64_t used, int64_t heads,

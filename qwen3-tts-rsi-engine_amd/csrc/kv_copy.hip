@@ -268,8 +268,9 @@ extern "C" int q3t_grow_arena(void *dst, const void *src, int64_t planes, int64_
         new_bytes < old_bytes || new_bytes < 1)
         return Q3T_EINVAL;
     if (old_bytes % 16 || new_bytes % 16 || !aligned(dst, 16) || !aligned(src, 16)) return Q3T_EUNSUPPORTED;
-    const int64_t limit = INT32_MAX, vectors = new_bytes / 16, chunks = (vectors + kRunChunk - 1) / kRunChunk;
-    if (planes > limit / slots || planes * slots > limit / heads || vectors > limit ||
+    // a launch has fewer than 2^32 threads
+    const int64_t limit = ((int64_t)1 << 24) - 1, vectors = new_bytes / 16, chunks = (vectors + kRunChunk - 1) / kRunChunk;
+    if (planes > limit / slots || planes * slots > limit / heads || vectors > INT32_MAX ||
         planes * slots * heads > limit / chunks)
         return Q3T_EUNSUPPORTED;
     const GrowParams p = {(char *)dst, (const char *)src, (uint32_t)chunks, (uint32_t)(old_bytes / 16), (uint32_t)vectors,

@@ -4,6 +4,8 @@ Drop-in for ``copy_packed_prefix`` (qwen3_tts_engine/packed_kv.py:6-31): the sam
 arguments, the same validation and ``ValueError`` raised before any device write; the copy
 itself is the ``q3t_copy_strided`` HIP kernel (bit-exact element copy, any strides).
 """
+import math
+
 import torch
 
 from . import _lib
@@ -74,4 +76,11 @@ def can_grow_blocks(dst: torch.Tensor, src: torch.Tensor) -> bool:
     return (dst.is_cuda and dst.numel() > 0 and src.numel() > 0 and dst.dtype == src.dtype and dst.is_contiguous()
             and src.is_contiguous() and dst.data_ptr() % 16 == 0 and src.data_ptr() % 16 == 0
             and (src.shape[-2] * size) % 16 == 0 and (dst.shape[-2] * size) % 16 == 0
-            and dst.numel() * dst.element_size() // 16 < 1 << 31)
+            and grow_launch_fits(math.prod(dst.shape[:-2]), dst.shape[-2] * size))
+
+
+def grow_launch_fits(blocks: int, block_bytes: int) -> bool:
+    """Whether one launch covers the blocks: 1024 16-byte vectors a workgroup of 256 threads, fewer
+    than 2^32 threads, 32-bit vector numbers within a block."""
+    vectors = block_bytes // 16
+    return vectors < 1 << 31 and blocks * -(-vectors // 1024) < 1 << 24

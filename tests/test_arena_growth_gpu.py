@@ -36,3 +36,22 @@ def test_growth(pkg, device, packed, head_dim, capacity, dtype, active):
         assert torch.equal(target, expected)
     if packed:
         assert new.keys[0].data_ptr() == new.packed.data_ptr()
+
+
+def test_growth_to_32_gib(pkg, device):
+    """Offsets past 32 bits of bytes and of vectors, every word compared."""
+    weight = torch.empty(1, device=device, dtype=torch.bfloat16)
+    reference = SimpleNamespace(parameters=lambda: iter([weight]), layers=[None],
+                                config=SimpleNamespace(num_key_value_heads=4, head_dim=128))
+    old = pkg.SlotArena(reference, 4, 1 << 21, packed_kv=True)
+    words = old.packed.view(torch.int64)
+    torch.arange(words.numel(), device=device, out=words.view(-1))
+    new = pkg.grow_arena(old, 1 << 21, active=3)
+    assert pkg.packed_kv.can_grow_blocks(new.packed, old.packed) and new.packed.nbytes == 32 << 30
+    for plane in range(2):
+        for slot in range(4):
+            for head in range(4):
+                block, source = new.packed[plane, slot, head], old.packed[plane, slot, head]
+                kept = block[:1 << 21].view(torch.int64)
+                assert torch.equal(kept, source.view(torch.int64)) if slot < 3 else not bool(kept.any())
+                assert not bool(block[1 << 21:].view(torch.int64).any())

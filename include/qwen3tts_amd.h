@@ -143,10 +143,10 @@ int q3t_rope_tables(const int64_t *positions, int64_t n, const float *inv_freq, 
  *   - chunked: each request's keys cut into chunks of 64-key blocks (at most `max_chunks`
  *     per request), one workgroup per (request, chunk, KV head); the default otherwise (the
  *     code predictor's 16-row caches, short arenas, few requests).  With max_chunks <= 0 and
- *     splits == 0, bf16 rows of 128 below 2048 keys, and unfused bf16 rows of 64 whose planes
- *     are short and few, run unsplit: one workgroup per (request, KV head).  Over bf16 rows of
- *     128 it stops at the last key that a request's mask shows: keys behind it are read only
- *     within that key's 16 rows and the first 256, and none reaches the output, whatever it holds.
+ *     splits == 0, bf16 rows of 128 below 2048 keys run unsplit: one workgroup per (request, KV
+ *     head).  Under a mask it stops at the last key that a request's mask shows: keys behind it
+ *     are read only within that key's 16 rows and the first 256, and none reaches the output,
+ *     whatever it holds.
  * A request covered by several workgroups (balanced, chunked) merges their partial softmax
  * states through `workspace`; the last workgroup to finish writes the output.
  *

@@ -55,15 +55,6 @@ constexpr int kDirectMaxCtx = 2048;    // longest context it takes (a mask row's
 constexpr int kDirectManyPairs = 64;   // (request, KV head) pairs from which its workgroups are smaller
 void direct_launch(const DecodeParams &p, int group, int tokens, bool fused, hipStream_t s);
 
-// The same for types that the MFMA kernels do not take (decode_whole.hip).  Measured, split / whole,
-// us: above a plane of 256 KiB one CU's share of the longest request loses to the split (fp32 rows of
-// 128, 16 requests over 2000 rows: 36.3 / 44.6; at 512 rows 17.2 / 14.9).  With one workgroup per CU
-// and every context far below the capacity (32 requests of 63 keys in 512 rows) it is 0.4 us slower.
-constexpr int kWholeMinCtx = 64;             // one block of keys needs no more waves
-constexpr int kWholeMaxPlane = 256 << 10;    // bytes of a head's key rows
-constexpr int kWholeMaxPairs = 256;          // one workgroup per CU
-void whole_launch(const DecodeParams &p, int group, int tokens, hipStream_t s);
-
 // 4 bytes per lane from global memory into LDS at lds_base + 4 * lane (the mask words of a
 // stage's rows); offsets past the resource's range write zeros.
 Q3T_DEVICE void load_to_lds4(i32x4_t rsrc, uint32_t voffset, uint32_t lds_base) {

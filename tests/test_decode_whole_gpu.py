@@ -1,8 +1,7 @@
-"""Decode attention of bf16 rows of 64 with one workgroup per (request, KV head) (few requests over
-arenas of 65 to 2047 rows), and of fp32 rows, which stay split, at the same sizes: against float64
-(fp32: 1e-5; bf16: max-abs <= 2e-2, mean-abs <= 2e-3) with lengths around the workgroup's blocks of
-128, 256 and 512 keys, invalid positions, one and two query tokens and masks; fp32 also against
-another number of chunks."""
+"""Decode attention over arenas of 65 to 2047 rows of the types that stay split (fp32, and bf16 rows of
+64): against float64 (fp32: 1e-5; bf16: max-abs <= 2e-2, mean-abs <= 2e-3) with lengths around 64, 128,
+256 and 512 keys, invalid positions, one and two query tokens and masks; fp32 also against another
+number of chunks."""
 import numpy as np
 import pytest
 import torch

@@ -47,6 +47,23 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kEmpty = -1.0e30f;  // finite "no key yet" running max
 constexpr int kMinShare = 32;       // balanced grid: fewest keys per workgroup
 
+// A call in which every request attends all of its keys has this array for its positions, so that the
+// kernels load a position as in any other call; they know it by its address.  (A branch on a null
+// pointer ahead of the load, with two argument loads behind it, cost an fp32 step of 16 requests
+// 1.2%; another argument to tell the calls apart 0.7%, its load taken ahead of the pointer's.)
+struct NoPositions {
+    int64_t v[kMaxBatch];
+    constexpr NoPositions() : v() {
+        for (int64_t &x : v) x = -1;
+    }
+};
+static __device__ NoPositions no_positions;
+
+// A request's keys, from its position: none where it is not one of the arena's.
+Q3T_DEVICE int keys_of(const DecodeParams &p, int64_t pos) {
+    return (uint64_t)pos < (uint64_t)(uint32_t)p.ctx ? (int)pos + 1 : p.pos == no_positions.v ? p.ctx : 0;
+}
+
 // Partial score of one lane: its 16 bytes of the query row and of the key row.
 template <typename T>
 Q3T_DEVICE float lane_dot(const U4 &q, const U4 &k) {
@@ -1536,10 +1553,10 @@ static int dispatch_sq(const DecodeParams &p, int sq, bool fused, hipStream_t s)
     if (fused) {
         if constexpr (sizeof(T) == 2 && D == 128) {
             if (sq == 1) {
-                if (p.mask) launch_decode<T, D, G, 1, true, true>(p, s);
+                if (p.has_mask) launch_decode<T, D, G, 1, true, true>(p, s);
                 else launch_decode<T, D, G, 1, true, false>(p, s);
             } else if (sq == 2) {
-                if (p.mask) launch_decode<T, D, G, 2, true, true>(p, s);
+                if (p.has_mask) launch_decode<T, D, G, 2, true, true>(p, s);
                 else launch_decode<T, D, G, 2, true, false>(p, s);
             } else {
                 return Q3T_EUNSUPPORTED;
@@ -1550,10 +1567,10 @@ static int dispatch_sq(const DecodeParams &p, int sq, bool fused, hipStream_t s)
         }
     }
     if (sq == 1) {
-        if (p.mask) launch_decode<T, D, G, 1, false, true>(p, s);
+        if (p.has_mask) launch_decode<T, D, G, 1, false, true>(p, s);
         else launch_decode<T, D, G, 1, false, false>(p, s);
     } else if (sq == 2) {
-        if (p.mask) launch_decode<T, D, G, 2, false, true>(p, s);
+        if (p.has_mask) launch_decode<T, D, G, 2, false, true>(p, s);
         else launch_decode<T, D, G, 2, false, false>(p, s);
     } else {
         return Q3T_EUNSUPPORTED;
@@ -1569,21 +1586,6 @@ static int dispatch_g(const DecodeParams &p, int g, int sq, bool fused, hipStrea
         case 4: return dispatch_sq<T, D, 4>(p, sq, fused, s);
         default: return Q3T_EUNSUPPORTED;
     }
-}
-
-// Memory that the positions of a call without any are loaded from (their values are not used), per
-// device; its address is looked up once.
-static __device__ int64_t no_positions[kMaxBatch];
-constexpr int kMaxDevices = 64;
-static const int64_t *any_positions() {
-    static std::mutex mutex;
-    static const int64_t *found[kMaxDevices];
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-    std::lock_guard<std::mutex> lock(mutex);
-    void *ptr = nullptr;
-    if (!found[dev] && hipGetSymbolAddress(&ptr, HIP_SYMBOL(no_positions)) == hipSuccess) found[dev] = (const int64_t *)ptr;
-    return found[dev];
 }
 
 // Host-side validation and parameter set-up shared by every decode entry point; the device
@@ -1633,6 +1635,7 @@ static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, Deco
     p.bundles = grid == Q3T_GRID_BUNDLED ? (int)bundle_count(a) : 0;
     p.stream = stream_kv(a->batch, a->kv_heads, a->ctx, a->head_dim * es);
     p.scale_log2 = a->scale * kLog2e;
+    p.has_mask = a->mask != nullptr;
     p.mask_dtype = (int)a->mask_dtype;
     p.q = (const char *)a->query;
     p.q_sb = a->q_stride_b; p.q_ss = a->q_stride_s; p.q_sh = a->q_stride_h;
@@ -1640,9 +1643,7 @@ static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, Deco
     p.k_sb = a->k_stride_b; p.k_sh = a->k_stride_h; p.k_st = a->k_stride_t;
     p.v_sb = a->v_stride_b; p.v_sh = a->v_stride_h; p.v_st = a->v_stride_t;
     p.offs = a->kv_offsets;
-    p.pos = a->positions;
-    if (all_keys && !(p.pos = any_positions())) return (int)hipErrorInvalidDevicePointer;
-    p.pos_limit = all_keys ? 0 : (int)a->ctx;
+    p.pos = all_keys ? nullptr : a->positions;
     p.mask = (const char *)a->mask;
     p.m_sb = a->mask_stride_b; p.m_ss = a->mask_stride_s; p.m_st = a->mask_stride_t;
     p.out = (char *)a->out;
@@ -1668,7 +1669,20 @@ static int decode_params(const q3t_decode_args *a, char *ws, bool all_keys, Deco
     return Q3T_OK;
 }
 
-static int decode_launch(const q3t_decode_args *a, const DecodeParams &p, void *stream) {
+constexpr int kMaxDevices = 64;
+// The device address of no_positions, looked up once per device.
+static const int64_t *all_keys_positions() {
+    static std::mutex mutex;
+    static const int64_t *found[kMaxDevices];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lock(mutex);
+    void *ptr = nullptr;
+    if (!found[dev] && hipGetSymbolAddress(&ptr, HIP_SYMBOL(no_positions)) == hipSuccess) found[dev] = (const int64_t *)ptr;
+    return found[dev];
+}
+
+static int decode_launch(const q3t_decode_args *a, DecodeParams &p, void *stream) {
     hipStream_t s = (hipStream_t)stream;
     const int g = (int)(a->q_heads / a->kv_heads);
     const int sq = (int)a->query_len;
@@ -1677,6 +1691,7 @@ static int decode_launch(const q3t_decode_args *a, const DecodeParams &p, void *
         direct_launch(p, g, sq, fused, s);
         return launch_status();
     }
+    if (!p.pos && !(p.pos = all_keys_positions())) return (int)hipErrorInvalidDevicePointer;
     int st;
     if (a->dtype == Q3T_BF16)
         st = a->head_dim == 128 ? dispatch_g<uint16_t, 128>(p, g, sq, fused, s)

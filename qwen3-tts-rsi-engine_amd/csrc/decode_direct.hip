@@ -563,7 +563,7 @@ void direct_launch(const DecodeParams &d, int group, int tokens, bool fused, hip
     p.scale_log2 = d.scale_log2; p.eps = d.eps;
     p.ctx = d.ctx; p.mask_dtype = d.mask_dtype; p.m_sb = d.m_sb; p.m_ss = d.m_ss; p.stream = d.stream;
     p.vec_out = ((reinterpret_cast<uintptr_t>(d.out) | p.o_sb | p.o_ss | p.o_sh) & 7) == 0;
-    const Call a = {d.B, d.Hkv, waves(d), d.mask != nullptr, d.qnw || d.knw, d.pos_limit ? d.pos : nullptr, stream};
+    const Call a = {d.B, d.Hkv, waves(d), d.has_mask != 0, d.qnw || d.knw, d.pos, stream};
     switch (group) {
         case 1: launch_tokens<1>(a, tokens, fused, p); break;
         case 2: launch_tokens<2>(a, tokens, fused, p); break;

@@ -12,13 +12,13 @@ struct DecodeParams {
     int splits;             // balanced grid: workgroups per KV head (0: chunked grid)
     int bundles;            // bundled grid: workgroups per KV head (0: another grid)
     float scale_log2;
-    int pos_limit, mask_dtype;  // pos_limit: see keys_of
+    int has_mask, mask_dtype;
     const char *q;
     int64_t q_sb, q_ss, q_sh;
     char *k, *v;
     int64_t k_sb, k_sh, k_st, v_sb, v_sh, v_st;
     const int64_t *offs;
-    const int64_t *pos;
+    const int64_t *pos;     // null: every request attends all of its keys
     const char *mask;
     int64_t m_sb, m_ss, m_st;
     char *out;
@@ -35,15 +35,6 @@ struct DecodeParams {
     int64_t nk_ss, nv_ss, cs_ss;  // fused, two tokens: token strides of new K/V and cos/sin
     const int32_t *plan;    // bundled grid: the step's plan (decode_plan.hip), null without one
 };
-
-// A request's keys, from its position: none where it is not one of the arena's.  A call in which every
-// request attends all of its keys has pos_limit 0 (else ctx) and some readable memory as `pos`, whose
-// content is not used: the position is loaded as in any other call.  (A branch on a null `pos` ahead
-// of the load, two argument loads behind it, cost an fp32 step of 16 requests 1.2%; selecting address
-// and value by bits 0.8%.)
-Q3T_DEVICE int keys_of(const DecodeParams &p, int64_t pos) {
-    return (uint64_t)pos < (uint64_t)(uint32_t)p.pos_limit ? (int)pos + 1 : p.ctx - p.pos_limit;
-}
 
 // The step plan (decode_plan.hip): bundles per KV head, plan size in int32 and its launch.
 int64_t plan_bundle_count(int64_t batch, int64_t kv_heads);

@@ -1389,6 +1389,8 @@ static bool bundle_ok(const q3t_decode_args *a) {
     return a->dtype == Q3T_BF16 && a->head_dim == 128 && a->query_len == 1 && bundle_mask_ok(a) &&
            a->batch <= kBundleMaxBatch && a->q_heads / a->kv_heads <= 4;
 }
+constexpr int64_t kDirectMaxPairs1 = 512, kDirectMaxPairs2 = 4096;  // of one and two query rows a key
+constexpr int64_t kDirectMaxCtx1 = 1024, kDirectFewPairs1 = 16;     // one query row
 // Whether a call on the chunked grid runs unsplit, one workgroup per (request, KV head)
 // (decode_direct.hip): bf16 rows of 128, one or two query tokens, row offsets that fit 32 bits;
 // a mask as the bundled grid takes it.  Callers that set a chunk count, or
@@ -1399,6 +1401,16 @@ static bool direct_ok(const q3t_decode_args *a) {
         a->ctx >= kDirectMaxCtx || a->splits != 0 || a->max_chunks > 0)
         return false;
     if (!bundle_mask_ok(a) || (a->mask && a->mask_stride_s < 0)) return false;
+    // Its workgroups hold a ring of LDS, two to a CU, where the split kernel's many small ones fill it.
+    // With one query row a key (or two) and very many pairs that is dearer, most with short contexts;
+    // nothing is lost over 32 rows (one wave a workgroup).  us per launch, split / unsplit: one row, 64
+    // requests x 8 heads (512 pairs) of 40 keys 6.1 / 5.6, 128 x 8 8.4 / 8.9, 400 x 8 18.5 / 21.7, of U[1, 100]
+    // 64 x 8 7.3 / 6.7, 400 x 8 20.9 / 23.9, of U[1, 500] 128 x 8 28.6 / 26.9; two rows, 500 x 8 of 40 keys
+    // 29.5 / 29.5, 1000 x 8 47.8 / 49.1.  And one row over long arenas, where the split shortens the longest
+    // request: 4 x 8 of U[1, 2000] 18.6 / 20.1, 4 x 8 of U[1, 1000] 17.8 / 9.6, 1 x 8 of 2000 24.0 / 14.6.
+    const int64_t row_count = G * a->query_len, pairs = a->batch * a->kv_heads;
+    if (a->ctx > kDirectOneWave && row_count <= 2 && pairs > (row_count == 1 ? kDirectMaxPairs1 : kDirectMaxPairs2)) return false;
+    if (row_count == 1 && a->ctx > kDirectMaxCtx1 && pairs > kDirectFewPairs1) return false;
     // the whole extent of the rows of a call in 31-bit byte offsets, key rows apart, arena planes in
     // 32-bit counts of 16 bytes
     const int64_t B = a->batch, S = a->query_len, Hq = a->q_heads, Hkv = a->kv_heads;

@@ -563,7 +563,8 @@ static void launch_tokens(const Call &a, int tokens, bool fused, const DirectPar
 // flight bound it; four from kDirectManyPairs, where two workgroups share a CU (us per layer, eight /
 // four waves: 4 requests of 100..500 keys 7.1 / 7.7, 8 of 30..511 9.0 / 8.3, 64 of them 17.9 / 15.4).
 static int waves(const DecodeParams &p) {
-    if (p.ctx <= 2 * kKeys) return 1;
+    static_assert(kDirectOneWave == 2 * kKeys, "two stages");
+    if (p.ctx <= kDirectOneWave) return 1;
     return (int64_t)p.B * p.Hkv >= kDirectManyPairs ? 4 : 8;
 }
 

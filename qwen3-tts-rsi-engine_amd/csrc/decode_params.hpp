@@ -43,6 +43,7 @@ int plan_launch(const int64_t *pos, int batch, int ctx, int bundles, int32_t *pl
 
 // The unsplit form of the chunked grid (decode_direct.hip): one workgroup per (request, KV head).
 constexpr int kDirectMaxCtx = 2048;    // longest context it takes (a mask row's words in LDS)
+constexpr int kDirectOneWave = 32;     // longest context of one wave a workgroup
 constexpr int kDirectManyPairs = 64;   // (request, KV head) pairs from which its workgroups are smaller
 void direct_launch(const DecodeParams &p, int group, int tokens, bool fused, hipStream_t s);
 

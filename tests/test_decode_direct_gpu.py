@@ -217,6 +217,19 @@ def test_step_in_a_graph_follows_rewritten_positions(pkg, device):
         assert torch.equal(out, expected) and torch.equal(keys, keys2) and torch.equal(values, values2)
 
 
+@pytest.mark.parametrize("batch,kv_heads,capacity,group,tokens,chunks", [
+    (65, 8, 40, 1, 1, 1), (3, 8, 1100, 1, 1, 18), (513, 8, 33, 2, 1, 1), (513, 8, 40, 1, 2, 1)])
+def test_many_pairs_of_few_rows_stay_split(pkg, device, batch, kv_heads, capacity, group, tokens, chunks):
+    """Calls past the unsplit form's lines: bit for bit the split kernel's with its own chunk count, and
+    one request fewer (or none past the line) as close to it."""
+    keys, values, q, _, _, positions = _problem(batch, kv_heads, group, capacity, 23, device, tokens)
+    positions = positions.clamp(tokens - 1, capacity - 1).to(device)
+    out = pkg.decode_attention(q, keys, values, positions)
+    assert torch.equal(out, pkg.decode_attention(q, keys, values, positions, max_chunks=chunks))
+    fewer = pkg.decode_attention(q[1:], keys[1:], values[1:], positions[1:])
+    assert_attention_close(f64(fewer), f64(out[1:]))
+
+
 @pytest.mark.parametrize("batch,capacity,dtype,head_dim", [
     (6, 300, torch.bfloat16, 128), (64, 1024, torch.bfloat16, 128), (4, 2100, torch.bfloat16, 128),
     (5, 200, torch.float32, 128), (5, 200, torch.bfloat16, 64)])

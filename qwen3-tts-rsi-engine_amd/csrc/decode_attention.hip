@@ -47,10 +47,11 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kEmpty = -1.0e30f;  // finite "no key yet" running max
 constexpr int kMinShare = 32;       // balanced grid: fewest keys per workgroup
 
-// A call in which every request attends all of its keys has this array for its positions, so that the
-// kernels load a position as in any other call; they know it by its address.  (A branch on a null
-// pointer ahead of the load, with two argument loads behind it, cost an fp32 step of 16 requests
-// 1.2%; another argument to tell the calls apart 0.7%, its load taken ahead of the pointer's.)
+// A call in which every request attends all of its keys has this array for its positions, and bit 0
+// of its pointer set, so that the kernels load a position as in any other call and need no other
+// argument to know it.  (A branch on a null pointer ahead of the load, with two argument loads behind
+// it, cost an fp32 step of 16 requests 1.2%; one more argument 0.7%, its load taken ahead of the
+// pointer's.)
 struct NoPositions {
     int64_t v[kMaxBatch];
     constexpr NoPositions() : v() {
@@ -59,9 +60,14 @@ struct NoPositions {
 };
 static __device__ NoPositions no_positions;
 
+Q3T_DEVICE int64_t position_of(const DecodeParams &p, int b) {
+    typedef __attribute__((address_space(4))) const int64_t constant_int64_t;
+    return ((constant_int64_t *)(reinterpret_cast<uintptr_t>(p.pos) & ~(uintptr_t)1))[b];
+}
 // A request's keys, from its position: none where it is not one of the arena's.
 Q3T_DEVICE int keys_of(const DecodeParams &p, int64_t pos) {
-    return (uint64_t)pos < (uint64_t)(uint32_t)p.ctx ? (int)pos + 1 : p.pos == no_positions.v ? p.ctx : 0;
+    const int others = reinterpret_cast<uintptr_t>(p.pos) & 1 ? p.ctx : 0;
+    return (uint64_t)pos < (uint64_t)(uint32_t)p.ctx ? (int)pos + 1 : others;
 }
 
 // Partial score of one lane: its 16 bytes of the query row and of the key row.
@@ -605,7 +611,7 @@ decode_chunks_kernel(DecodeParams p) {
     const int rest = blockIdx.x / p.Hkv;
     const int c = rest % p.nchunks, b = rest / p.nchunks;
 
-    const int64_t pb = p.pos[b];
+    const int64_t pb = position_of(p, b);
     Work work;
     work.load_rows(p, b, h);
     const int L = keys_of(p, pb);
@@ -678,7 +684,7 @@ decode_balanced_kernel(DecodeParams p) {
             const int b = tid * per + e;
             w[e] = 0;
             if (e < per && b < p.B) {
-                const int64_t pb = p.pos[b];
+                const int64_t pb = position_of(p, b);
                 const int L = keys_of(p, pb);
                 sm_len[b] = L;
                 w[e] = L > 0 ? L : 1;
@@ -925,7 +931,7 @@ __global__ void __launch_bounds__(kThreads) decode_bundled_kernel(const int32_t 
         int64_t pb[2] = {-1, -1};
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-            if (lane + 64 * e < p.B) pb[e] = p.pos[lane + 64 * e];
+            if (lane + 64 * e < p.B) pb[e] = position_of(p, lane + 64 * e);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int b = lane + 64 * e;
@@ -1703,7 +1709,11 @@ static int decode_launch(const q3t_decode_args *a, DecodeParams &p, void *stream
         direct_launch(p, g, sq, fused, s);
         return launch_status();
     }
-    if (!p.pos && !(p.pos = all_keys_positions())) return (int)hipErrorInvalidDevicePointer;
+    if (!p.pos) {
+        const int64_t *positions = all_keys_positions();
+        if (!positions) return (int)hipErrorInvalidDevicePointer;
+        p.pos = reinterpret_cast<const int64_t *>(reinterpret_cast<uintptr_t>(positions) | 1);
+    }
     int st;
     if (a->dtype == Q3T_BF16)
         st = a->head_dim == 128 ? dispatch_g<uint16_t, 128>(p, g, sq, fused, s)

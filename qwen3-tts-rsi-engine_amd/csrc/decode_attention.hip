@@ -1360,23 +1360,27 @@ static int64_t chunk_count(int64_t batch, int64_t kv_heads, int64_t ctx, int64_t
 // The grid a call runs on (Q3T_GRID_CHUNKED, _BALANCED or _BUNDLED; -1: a requested grid the
 // call does not qualify for).  The bundled grid needs bf16 rows of 128, one query token, at
 // most kBundleMaxBatch requests, q_heads / kv_heads <= 4, and a mask with unit key stride.
-// Automatic choice, measured (bf16, 16/8 heads, 28-layer graphs of fused steps, us per layer).
-// The bundled grid pairs long requests with short ones, so it wins on ragged contexts; with
-// equal contexts two whole requests per workgroup lose to the chunked grid's one per
-// workgroup, two workgroups per CU (64 requests of 512 keys in a 1024-row arena: 27.2 against
-// 26.5; of 64 keys in a 512-row arena: 10.9 against 8.1).  The host sees the capacity, not
+// Automatic choice, measured (bf16, 16/8 heads, graphs of fused steps, us per layer; chunked runs
+// unsplit below 2048 rows).  The bundled grid pairs long requests with short ones, so it wins on
+// ragged contexts of many requests; with equal contexts two whole requests per workgroup lose to the
+// unsplit form's one per workgroup, two workgroups per CU (64 requests of 512 keys in a 1024-row arena:
+// 25.2 against 24.6; of 64 keys in a 512-row arena 9.3 against 6.7).  The host sees the capacity, not
 // the lengths, so:
-//  - 24..63 requests (192..511 (request, KV head) items) from 512 rows: bundled, which beat
-//    the chunked grid on every distribution measured (32 requests of 64 keys: 7.9 against
-//    11.0; 32 over 512 rows, uniform lengths: 13.5 against 16.7; 24 over 1024 rows: 19.4
-//    against 21.7 balanced);
-//  - 64..128 requests from 1024 rows (the talker step's ragged contexts: 26.1 against 30.3
-//    chunked; 96 requests over 2048 rows: 71.7 against 78.2 balanced);
+//  - 24..63 requests (192..511 (request, KV head) items) from 512 rows: bundled.  The line was drawn
+//    against the split kernel (32 over 512 rows 16.7, of 64 keys 11.0) and balanced (24 over 1024 rows
+//    21.5).  Against the unsplit form it holds for 40 and more (40 over 1024 rows, uniform lengths: 21.0
+//    bundled, 22.7 unsplit; 48: 22.2 / 23.9, over 2000 rows 41.0 / 47.9, over 512 rows 14.8 / 14.6) and not
+//    for 24..32 (32 over 512 rows 12.9 / 10.5, of 64 keys 6.4 / 5.0, over 1024 rows 19.6 / 17.2, over 2000
+//    rows 33.6 / 30.3; 24 over 1024 rows 18.9 / 15.8), which keep the grid that their plans, names and
+//    workspaces are for;
+//  - 64..128 requests from 1024 rows (the talker step's ragged contexts: 26.4 against 28.4 unsplit;
+//    128 requests 44.6 / 49.6; 96 requests over 2000 rows 67.6 / 68.9, 72.2 balanced);
 //  - from 4096 rows only with 384 items or more, where one or two whole requests per
 //    workgroup leave the longest unbalanced (32 requests: 60.9 against 52.9 balanced);
-//  - chunked below 512 rows (64 requests over 256 rows: 12.6 against 12.9 bundled) and for 64
+//  - chunked below 512 rows (64 requests over 256 rows: 10.7 unsplit, 12.7 bundled) and for 64
 //    or more requests over 512..1023 rows (the reference's valid-length probes, equal
-//    contexts); balanced otherwise from 2048 rows.
+//    contexts; 128 over 512 rows 27.4 / 28.3, of 64 keys 11.0 / 13.7); balanced otherwise from 2048 rows (8
+//    requests over 2100 rows 18.9, 23.7 chunked).
 constexpr int64_t kBundleMinCtx = 512;
 constexpr int64_t kBundleMinItems = 192;
 constexpr int64_t kBundleManyItems = 512;      // 64 requests of 8 KV heads

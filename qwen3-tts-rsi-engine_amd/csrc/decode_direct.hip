@@ -25,8 +25,8 @@
 // per M0 write and address arithmetic placed under the loads' latency took the 16-row launch
 // from 6.2 to 3.8 us.
 // Measured, us per layer (28-layer graphs of fused steps, 16/8 heads), split kernel -> this one:
-// 64 requests x 16 rows 6.5 -> 3.8; 1 x 300 keys 10.7 -> 6.5; 21 x 30..511 keys 16.6 -> 9.4;
-// 64 x 32..511 keys 18.0 -> 15.4; 128 x 512 rows 32.0 -> 28.1; 1 x 1750 keys 22.5 -> 11.9.
+// 64 requests x 16 rows 6.5 -> 3.8; 1 x 300 keys 10.7 -> 6.1; 21 x 30..511 keys 16.6 -> 9.2;
+// 64 x 32..511 keys 18.0 -> 15.7; 128 x 32..512 keys 32.0 -> 26.6; 1 x 1750 keys 22.5 -> 13.4.
 //   * masked launches bring the request's whole mask row into LDS once and stop at its last
 //     visible key.  Each wave's first two stages are on their way before the mask is looked at, so
 //     of the keys that the mask hides behind it, those stages' are read and no others; none reaches
@@ -561,7 +561,8 @@ static void launch_tokens(const Call &a, int tokens, bool fused, const DirectPar
 // Waves per workgroup.  One where the arena's rows are one or two stages of a wave (the code
 // predictor's 16-row caches): no merge.  Eight for a few pairs, where a workgroup's own loads in
 // flight bound it; four from kDirectManyPairs, where two workgroups share a CU (us per layer, eight /
-// four waves: 4 requests of 100..500 keys 7.1 / 7.7, 8 of 30..511 9.0 / 8.3, 64 of them 17.9 / 15.4).
+// four waves: one request of 1750 keys 13.4 / 17.8, 4 of 100..500 7.4 / 7.9, 8 of 30..511 9.0 / 8.5, 64 of
+// them 18.4 / 15.8).
 static int waves(const DecodeParams &p) {
     static_assert(kDirectOneWave == 2 * kKeys, "two stages");
     if (p.ctx <= kDirectOneWave) return 1;

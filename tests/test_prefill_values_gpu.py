@@ -1,6 +1,6 @@
 """Prefill with the values read from the projection's rows: the prologue writes only the
 rotated keys (``prefill_rope_write(value=None)``) and the attention launch reads each key's
-value from the step's own value rows while its copy workgroups write those rows into the
+value from the step's own value rows while its workgroups write those rows into the
 arena (``prefill_attention(new_values=...)``).
 
 Every case is compared bit for bit with the two-launch path that writes keys and values in
@@ -75,8 +75,7 @@ def test_values_past_the_capacity_are_not_copied(pkg, device, group, head_dim):
 
 
 def test_more_than_64_requests(pkg, device):
-    """70 requests: the copy workgroups find a token's request by a search of the row
-    offsets instead of one ballot."""
+    """70 requests: the work items are numbered over a padded grid instead of by ballots."""
     lengths = (torch.arange(70) * 7 % 61 + 1).tolist()
     kv_slots = torch.randperm(80, generator=torch.Generator().manual_seed(5))[:70].to(device)
     _both(pkg, lengths, 16, 8, 128, 80, 64, 21, device, kv_slots=kv_slots)

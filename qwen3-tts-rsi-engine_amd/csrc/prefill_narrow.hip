@@ -50,15 +50,16 @@ prefill_narrow_kernel(const int32_t *cu, const int64_t *slots, int nb, PrefillPa
     const bool copies = (int)blockIdx.x >= p.attn_wgs;  // past the attention grid: value rows to copy
     const int wg = copies ? (int)blockIdx.x - p.attn_wgs : place_workgroup(blockIdx.x, p.attn_wgs);
     const int h = wg % p.Hq, rest = wg / p.Hq;
-    if (copies && rest == 0) copy_rows_past_the_end<D, false>(p, cu, slots, nb, start, next, h);
+    if (copies && wg >= p.attn_wgs) {  // past these: rows that no block covers
+        copy_other_rows<D, false>(p, cu, slots, nb, wg - p.attn_wgs, (int64_t)p.nqb * kQBlock);
+        return;
+    }
     PrefillItem item;
     if (!find_item<kQBlock>(p, cu, slots, nb, start, next, slot_l, rest, item)) return;
     const int b = item.b, t0 = item.t0, n = item.n, kn = item.kn, q0 = item.qb * kQBlock;
     const int64_t slot = item.slot;
     if (copies) {
-        // the last block copies the rows of a request longer than max_seqlen as well
-        const int end = item.qb == p.nqb - 1 ? n : min(n, q0 + kQBlock);
-        copy_uncovered_rows<D, false>(p, h, slot, t0, q0, (int64_t)t0 + end);
+        copy_uncovered_rows<D, false>(p, h, slot, t0, q0, (int64_t)t0 + min(n, q0 + kQBlock));
         return;
     }
     // keys 0 ... kv_end-1 are visible to this block; the arena holds at most `cap` of them.
@@ -318,7 +319,7 @@ void launch_prefill_narrow(const PrefillParams &p, int64_t head_dim, int64_t max
     q.nqb = (int)((max_seqlen + kQBlock - 1) / kQBlock);
     q.by_request = 0;
     q.attn_wgs = (int)prefill_workgroups(p, kQBlock, p.Hq, max_seqlen);
-    const dim3 grid((uint32_t)(p.nv ? 2 * q.attn_wgs : q.attn_wgs));
+    const dim3 grid((uint32_t)(p.nv ? 2 * q.attn_wgs + other_row_workgroups(p) : q.attn_wgs));
     if (head_dim == 128) launch<128>(q, grid, s);
     else launch<64>(q, grid, s);
 }

@@ -58,6 +58,9 @@ inline int64_t prefill_workgroups(const PrefillParams &p, int64_t block, int64_t
     return bound < wgs ? bound : wgs;
 }
 
+// Workgroups that look for rows that no query block covers (copy_other_rows), with new rows.
+inline int64_t other_row_workgroups(const PrefillParams &p) { return p.nv ? (int64_t)p.Hkv * ((p.B + 63) / 64) : 0; }
+
 // The form for one-head groups in launches of few workgroups (prefill_narrow.hip).
 void launch_prefill_narrow(const PrefillParams &p, int64_t head_dim, int64_t max_seqlen, hipStream_t s);
 
@@ -93,6 +96,7 @@ template <int D, bool RK>
 Q3T_DEVICE void copy_uncovered_rows(const PrefillParams &p, int h, int64_t slot, int t0, int pos0, int64_t t1) {
     constexpr int HALF = D / 16;  // chunks of half a row
     const int64_t end = min(t1 - t0, p.cap);
+#pragma unroll 1
     for (int64_t pos = (int64_t)pos0 + threadIdx.x / HALF; pos < end; pos += 256 / HALF) {
         const int ch = threadIdx.x % HALF;
         const int64_t t = t0 + pos;
@@ -112,15 +116,30 @@ Q3T_DEVICE void copy_uncovered_rows(const PrefillParams &p, int h, int64_t slot,
     }
 }
 
-// Tokens past the last request's end go on at its next positions.  `start`, `next`: the lane's
-// request's first token and the next one's (up to 64 requests).
+// Work item `item` of the rows that no query block covers, of a KV head and up to 64 requests: rows of
+// requests longer than `covered`, and the tokens past the last request's end, which go on at its next
+// positions.
 template <int D, bool RK>
-Q3T_DEVICE void copy_rows_past_the_end(const PrefillParams &p, const int32_t *cu, const int64_t *slots, int nb, int start, int next, int h) {
-    const int last = nb - 1;
-    const int from = nb <= 64 ? __builtin_amdgcn_readlane(start, last) : cu[last];
-    const int past = nb <= 64 ? __builtin_amdgcn_readlane(next, last) : cu[nb];
-    if (__builtin_expect(past < p.T && past >= from && from >= 0, false))
-        copy_uncovered_rows<D, RK>(p, h, slots ? slots[last] : last, from, past - from, p.T);
+Q3T_DEVICE void copy_other_rows(const PrefillParams &p, const int32_t *cu, const int64_t *slots, int nb, int item, int64_t covered) {
+    const int h = item % p.Hkv, b0 = item / p.Hkv * 64, lane = threadIdx.x & 63;
+    int t0 = -1, t1 = -1;
+    if (b0 + lane < nb) {
+        t0 = cu[b0 + lane];
+        t1 = cu[b0 + lane + 1];
+    }
+    const int64_t rows = t0 < 0 || t0 >= p.T ? 0 : min((int64_t)t1 - t0, p.T - t0);
+    const int last = nb - 1 - b0;  // the last request's lane, past 63 in an earlier item
+    const bool past = lane == last && t0 >= 0 && t1 >= t0 && t1 < p.T;
+    uint64_t longer = __builtin_amdgcn_ballot_w64(rows > covered), open = __builtin_amdgcn_ballot_w64(past);
+    // a request longer than covered from there to its end; then the last one from its end on
+    while (longer | open) {
+        const int l = __builtin_ctzll(longer ? longer : open), b = b0 + l;
+        const int from = __builtin_amdgcn_readlane(t0, l), end = __builtin_amdgcn_readlane(t1, l);
+        const int64_t slot = slots ? slots[b] : b;
+        copy_uncovered_rows<D, RK>(p, h, slot, from, longer ? (int)covered : end - from, longer ? min((int64_t)end, p.T) : p.T);
+        if (longer) longer &= longer - 1;
+        else open = 0;
+    }
 }
 
 // Placement: the hardware deals workgroup i to XCD i % 8 and, within an XCD, to its 32 CUs

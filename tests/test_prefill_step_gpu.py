@@ -107,6 +107,7 @@ def test_a_request_longer_than_max_seqlen_leaves_the_others_whole(pkg, device, l
 @pytest.mark.parametrize("group", [1, 2, 4])
 @pytest.mark.parametrize("lengths,max_seqlen,past,capacity", [
     ([20, 30], 32, 7, 64), ([200, 40, 0], 40, 3, 160), ([0], 8, 5, 16), ([30] * 70, 16, 90, 128),  # one launch
+    ([70] * 64, 60, 9, 96), ([70] * 65, 60, 9, 96), ([70] * 128, 64, 9, 96),   # 64 requests a workgroup
     ([300, 100, 130], 128, 70, 260), ([150] + [126] * 60, 128, 1, 512), ([300] * 70, 100, 9, 320)])
 def test_every_token_reaches_the_arena(pkg, device, lengths, max_seqlen, past, capacity, group, head_dim):
     """Tokens of requests longer than ``max_seqlen`` and past the last request's end: the arena bit for

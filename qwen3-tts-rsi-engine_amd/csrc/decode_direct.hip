@@ -127,6 +127,7 @@ Q3T_DEVICE void load_row16(const char *base, uint32_t voffset, uint32_t lds_base
 #define Q3T_GLOBAL __attribute__((address_space(1)))
 Q3T_DEVICE void global_store16(char *p, const U4 &v) { *(Q3T_GLOBAL i32x4_t *)(uintptr_t)p = __builtin_bit_cast(i32x4_t, v); }
 Q3T_DEVICE void global_store2(char *p, uint32_t v) { *(Q3T_GLOBAL uint16_t *)(uintptr_t)p = (uint16_t)v; }
+Q3T_DEVICE void global_store4(char *p, uint32_t v) { *(Q3T_GLOBAL uint32_t *)(uintptr_t)p = v; }
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 Q3T_DEVICE void global_store8(char *p, uint32_t lo, uint32_t hi) { *(Q3T_GLOBAL u32x2_t *)(uintptr_t)p = u32x2_t{lo, hi}; }
 
@@ -469,27 +470,38 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
             lds_write16(state ^ (db * 64), __builtin_bit_cast(U4, acc[db]));
     }
     lds_barrier();
-    const int outputs = R * 32;  // of four dims
-    for (int t = tid; t < outputs; t += W * 64) {
-        const int r = t / 32, d = t % 32 * 4;
-        const uint32_t from = lds(&s.ring[0][0][0]);
-        // a wave's four sums: the parts of the weights added up (unless a sum is infinite, whose
+    // The merge: V dims of a query row per thread.  With eight waves so few that all threads take one
+    // pass: four dims each, one wave at work for two rows, added up eight waves' three parts in 1-2% of a
+    // launch more (28 layers, one request of 200..400 keys 173.4 us, now 171.1).  With four it is the same.
+    constexpr int V = W < 8 || 2 * R / W >= 4 ? 4 : 2 * R / W >= 2 ? 2 : 1;
+    for (int t = tid; t < R * 128 / V; t += W * 64) {
+        const int r = t / (128 / V), d = t % (128 / V) * V;
+        const uint32_t from = lds(&s.ring[0][0][0]) + d % 4 * 4;
+        // a wave's sums: the parts of the weights added up (unless a sum is infinite, whose
         // remainder may be 0 x inf)
-        auto sums = [&](int w) {
-            auto column = [&](int c) {
-                return __builtin_bit_cast(f32x4_t, lds_read16(from + w * kStage + c * 512 + ((t % 32) ^ c) * 16));
+        auto sums = [&](int w, float (&x)[V]) {
+            auto column = [&](int c, float (&v)[V]) {
+                typedef float floats_t __attribute__((ext_vector_type(V)));
+                const floats_t f = *(__attribute__((address_space(3))) const floats_t *)(uintptr_t)(
+                    from + w * kStage + c * 512 + ((d / 4) ^ c) * 16);
+                __builtin_memcpy(v, &f, sizeof(v));
             };
-            f32x4_t a = column(r), rest = column(r + R);
-            if constexpr (THIRD) rest += column(r + 2 * R);
+            float rest[V];
+            column(r, x);
+            column(r + R, rest);
+            if constexpr (THIRD) {
+                float third[V];
+                column(r + 2 * R, third);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = __builtin_fabsf(a[i]) < INFINITY ? a[i] + rest[i] : a[i];
-            return a;
+                for (int i = 0; i < V; ++i) rest[i] += third[i];
+            }
+#pragma unroll
+            for (int i = 0; i < V; ++i) x[i] = __builtin_fabsf(x[i]) < INFINITY ? x[i] + rest[i] : x[i];
         };
-        float sl;
-        f32x4_t sa;
+        float sl, sa[V];
         if constexpr (W == 1) {
             sl = s.ml[0][r][1];
-            sa = sums(0);
+            sums(0, sa);
         } else {
             auto merge = [&](auto count) {
                 constexpr int N = decltype(count)::value;
@@ -497,12 +509,16 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
 #pragma unroll
                 for (int w = 1; w < N; ++w) mm = fmaxf(mm, s.ml[w][r][0]);
                 sl = 0.f;
-                sa = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < V; ++i) sa[i] = 0.f;
 #pragma unroll
                 for (int w = 0; w < N; ++w) {
                     const float wt = fexp2(s.ml[w][r][0] - mm);
+                    float x[V];
+                    sums(w, x);
                     sl += s.ml[w][r][1] * wt;
-                    sa += sums(w) * wt;
+#pragma unroll
+                    for (int i = 0; i < V; ++i) sa[i] += x[i] * wt;
                 }
             };
             // waves past the keys hold nothing
@@ -511,15 +527,22 @@ decode_direct_kernel(const int64_t *pos, DirectParams) {
         }
         const float inv = __builtin_amdgcn_rcpf(sl);
         char *o = out + ((r / G) * p.o_ss + (r % G) * p.o_sh + d * 2);
-        const uint2 w = {cvt_pk_bf16_canon(sa[0] * inv, sa[1] * inv), cvt_pk_bf16_canon(sa[2] * inv, sa[3] * inv)};
-        if (p.vec_out) {
-            global_store8(o, w.x, w.y);
-        } else {
-            global_store2(o, w.x);
-            global_store2(o + 2, w.x >> 16);
-            global_store2(o + 4, w.y);
-            global_store2(o + 6, w.y >> 16);
+        uint32_t y[(V + 1) / 2];
+#pragma unroll
+        for (int i = 0; i < V; i += 2) y[i / 2] = cvt_pk_bf16_canon(sa[i] * inv, sa[V > 1 ? i + 1 : 0] * inv);
+        if constexpr (V == 4) {
+            if (p.vec_out) {
+                global_store8(o, y[0], y[1]);
+                continue;
+            }
+        } else if constexpr (V == 2) {
+            if (p.vec_out) {
+                global_store4(o, y[0]);
+                continue;
+            }
         }
+#pragma unroll
+        for (int i = 0; i < V; ++i) global_store2(o + 2 * i, i % 2 ? y[i / 2] >> 16 : y[i / 2]);
     }
 }
 
